@@ -18,30 +18,30 @@
 //      of p in any order.
 //
 // The buffer is split into lane segments of kFnvLaneBytes bytes, a workgroup's 256 lanes covering 64 KiB, and the
-// low byte is resolved in three levels: bits 0-2, 3-5 and 6-7.  A level's map of a run of bytes takes the level's bits
+// low byte is resolved in levels: bits 0-3 and 4-7, or, where no workgroup waits for another (a check given carries),
+// bits 0-2, 3-5 and 6-7.  A level's map of a run of bytes takes the level's bits
 // at the run's start to their values at its end, given the true lower bits.  The term of a bit depends only on the
 // lower start bits, so the end value of a bit in a machine started from the true lower bits, with the bit itself 0,
 // is the run's term for that bit.  The top two bits of a level need no machines of their own: flipping start bit i
 // (the bits below it fixed) flips bit i at every position, which changes the term of bit i + 1 by the xor over the run
 // of 1 ^ y_i, y_i being bit i of ((l ^ b) mod 2^i) * 179; and y_i = l_i ^ l'_i ^ b_i, so that xor is
 //     (length mod 2) ^ (term of bit i) ^ (parity of bit i over the run's bytes).
-// A level for bits j .. j + k - 1 therefore runs 2^(k-2) machines (one per value of the unknown start bits
-// j .. j + k - 3): two for a three-bit level (start bit j = 0, 1) and one for a two-bit level.  Each lane runs its
-// segment as two halves of 128 bytes side by side: both halves' machines share the multiplies (two 8-bit machines per
-// 24-bit multiply, bytes 0 and 2; the first level needs only bits 0..2, which follow l' = (l ^ b) * 3 mod 8, so four
-// machines share one register a byte each), each half's map comes from its machines and its byte parities, and the
+// A level for bits j .. j + k - 1 therefore runs 2^(k-2) machines, one per value of the unknown start bits
+// j .. j + k - 3.  Each lane runs its segment as two halves of 128 bytes side by side: both halves' machines share the
+// multiplies (two 8-bit machines per 24-bit multiply, bytes 0 and 2; the lowest bits follow l' = (l ^ b) * 3 mod 16, so
+// four machines share one register a byte each), each half's map comes from its machines and its byte parities, and the
 // lane's map is the second half's after the first's.  Per level: the lanes ballot their maps, each workgroup forms
 // its map of the k-bit state from them, finds its start state by a look-back over the workgroups before it, each
-// lane derives its start bits from the workgroup's state and the ballots by xor-prefix arithmetic, and its first
-// half's map gives the bits at its midpoint.  After the third level every lane runs the full machine of both halves
-// from their now complete start bytes and forms its segment's Horner sum, scaled by p^(bytes after the segment); the
-// workgroups' sums are added, and a last kernel adds h_0 p^N.  All of it is one kernel that reads the input once (the
-// one-pass hash, below).
+// lane derives its start bits from the workgroup's state and the ballots by counting the lanes before it, and its first
+// half's map gives the bits at its midpoint.  After the last level every lane runs the full machine of both halves
+// from their now complete start bytes, whose products the matrix cores sum with the powers of p; the workgroups' sums are
+// added, and a last kernel adds h_0 p^N.  All of it is one kernel that reads the input once (the one-pass hash, below).
 #include <hip/hip_runtime.h>
 
 #include <atomic>
 #include <cstdint>
 #include <mutex>
+#include <type_traits>
 
 #include "sc_handoff.h"
 #include "sc_internal.hpp"
@@ -83,88 +83,154 @@ __device__ __forceinline__ void load_segment(const uint8_t* p, uint32_t (&w)[kFn
 __device__ __forceinline__ uint32_t step_pair(uint32_t x, uint32_t bb) {
     return __umul24((x ^ bb) & 0x00FF00FFu, kPrimeLow);
 }
-// Packed 16-bit subtraction of the two halves of a word (v_pk_sub_i16).
-typedef short v2i16 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t pk_sub(uint32_t a, uint32_t b) {
-    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2i16, a) - __builtin_bit_cast(v2i16, b));
-}
-
-// The Horner sum of a run of bytes is sum over c of d_c p^(len - c), d_c = (l ^ b) - l.  Each power of p is written
-// as four signed 16-bit digits (balanced base 2^16: p^k = sum_j digit_j 2^(16 j) mod 2^64, every digit in
-// [-2^15, 2^15); the carry out of the top digit is a multiple of 2^64 and drops), so per digit j the sum
-// S_j = sum_c d_c digit_j is exact in 32 bits (|d| <= 255), and two d values packed as signed 16-bit halves take one
-// packed dot product (v_dot2_i32_i16) per digit.
-__device__ __forceinline__ int32_t dot2(uint32_t a, uint32_t b, int32_t acc) {
-    return __builtin_amdgcn_sdot2(__builtin_bit_cast(v2i16, a), __builtin_bit_cast(v2i16, b), acc, false);
-}
-// sum_j S_j 2^(16 j) mod 2^64.
-__device__ __forceinline__ uint64_t digit_sum(int32_t s0, int32_t s1, int32_t s2, int32_t s3) {
-    return uint64_t(int64_t(s0)) + (uint64_t(int64_t(s1)) << 16) + (uint64_t(int64_t(s2)) << 32) +
-           (uint64_t(int64_t(s3)) << 48);
-}
-
-// Byte k of `a` in byte 0 and byte k of `b` in byte 2, zeros elsewhere (v_perm_b32: selector 0x0c gives a zero byte).
-__device__ __forceinline__ uint32_t pair_byte(uint32_t a, uint32_t b, int k) {
-    return __builtin_amdgcn_perm(b, a, uint32_t(k) | 0x0c00u | (uint32_t(4 + k) << 16) | 0x0c000000u);
-}
-
-// A lane's segment is summed as two halves of 128 bytes, their machines side by side in one register: the true low
-// bytes of their states sit in the low bytes of the halves of `m` (half A low, half B high, each half's high byte 0).
-// Per step one permute lines up a byte of each, one xor, one packed subtract gives both d values (A's in the low
-// half), one 24-bit multiply and a mask the next low bytes (the masked byte A's product stays below bit 16, as in
-// step_pair).  Byte c of B is weighted by p^(128 - c) and byte c of A by p^(256 - c), so each digit sum takes one
-// packed dot product per step against a word holding both digits, and the one sum is the segment's Horner sum
-// relative to its end (|S_j| < 128 * 2 * 255 * 2^15 < 2^31 stays exact).  About 4 VALU operations per byte, against
-// 7.5 for one byte at a time.
+// A segment's words as its passes read them: word k of half A and word k of half B become one word of their bytes 0
+// and 1 and one of their bytes 2 and 3, [a0 a1 b0 b1] and [a2 a3 b2 b3].  The bytes of an even step then lie in bytes 0
+// and 2 of a word, where the machines' states are, and those of an odd step one shift by 8 away: one operation per four
+// bytes in each pass, where picking the two bytes of every step out of the plain words took two.
 constexpr int kPairBytes = 128, kHalfWords = kPairBytes / 4;
+__device__ __forceinline__ uint32_t low_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
+__device__ __forceinline__ uint32_t high_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+// Its own inverse on the pairs: plain words to step words and back.
+__device__ __forceinline__ void pair_words(uint32_t (&w)[kFnvLaneBytes / 4]) {
+#pragma unroll
+    for (int k = 0; k < kHalfWords; ++k) {
+        const uint32_t a = w[k], b = w[kHalfWords + k];
+        w[k] = low_halves(a, b);
+        w[kHalfWords + k] = high_halves(a, b);
+    }
+}
+
+// Makes the words new to the compiler: it would otherwise compute each word's shift once and keep it, 64 more registers,
+// from one pass to the next (68 spilled words).
+__device__ __forceinline__ void renew_words(uint32_t (&w)[kFnvLaneBytes / 4]) {
+#pragma unroll
+    for (int k = 0; k < kFnvLaneBytes / 4; ++k) asm volatile("" : "+v"(w[k]));
+}
+
+// ---- the sum on the matrix cores -------------------------------------------------------------------------------------
+// A run of bytes adds sum over n of d_n p^(E_n) to the hash, d_n = x_n - l_n, x_n = l_n ^ b_n, E_n the bytes from n to
+// the input's end.  The machine's product 179 x_n = lo_n + 256 hi_n holds both: lo_n is l_(n+1), and
+// x_n = (lo_n + 256 hi_n) / 179, exact as a multiplication by the inverse of 179 modulo 2^64.  So
+//     sum d_n p^(E_n) = sum lo_n u(E_n) + sum hi_n v(E_n) + (low byte after the run) p^(E_end) - (low byte before) p^(E_0),
+//     u(E) = p^E / 179 - p^(E-1),   v(E) = 256 p^E / 179   (mod 2^64),
+// linear in the bytes of the products a lane's two machines leave in one register per step.  With the weights as eight
+// signed base-256 digits (balanced, so |digit| <= 128; the carry out of the top digit is a multiple of 2^64 and drops)
+// it is a product of 8-bit matrices: v_mfma_i32_16x16x64_i8, four steps' products per lane as A, the digits as B.  The
+// products' bytes are offset by -128 (one xor) to be signed, which adds a constant.  Row i of the result sums lanes
+// i, i + 16, i + 32, i + 48, whose distance is in the weights, and column j digit j; columns 0-7 hold the weights of an
+// even word and columns 8-15 those of the odd word after it, so one B serves two multiplications.  Every sum is below
+// 1024 * 2^14 in magnitude, so exact in 32 bits.
+// Against two packed 16-bit dot products per byte pair and digit (v_dot2_i32_i16, four 16-bit digits, 9 operations per
+// two bytes) this leaves the vector units four operations per two bytes.
 constexpr uint64_t prime_pow_of(uint64_t e) {
     uint64_t r = 1, b = kFnvPrime;
     for (; e; e >>= 1, b *= b)
         if (e & 1) r *= b;
     return r;
 }
-// p^(256 (63 - l)) for lane l: a lane's sum, relative to the end of its segment B, times this is relative to the end of
-// the wave's last segment B.
-struct LanePow {
-    uint64_t v[64];
-};
-constexpr LanePow lane_pow() {
-    LanePow t{};
-    for (int l = 0; l < 64; ++l) t.v[l] = prime_pow_of(uint64_t(kFnvLaneBytes) * uint64_t(63 - l));
-    return t;
+constexpr uint64_t inverse_of(uint64_t a) {   // modulo 2^64, a odd: Newton's iteration doubles the correct bits
+    uint64_t x = a;
+    for (int i = 0; i < 6; ++i) x *= 2u - a * x;
+    return x;
 }
-__constant__ LanePow kLanePow = lane_pow();
-struct HalfDigits {
-    uint32_t w[kPairBytes][4];   // [c][j]: digit j of p^(256 - c) in the low half, of p^(128 - c) above
+constexpr uint64_t kInv179 = inverse_of(kPrimeLow);
+static_assert(kInv179 * kPrimeLow == 1u, "the inverse of 179 modulo 2^64");
+constexpr uint64_t kPrimeInv = inverse_of(kFnvPrime);
+// u(E) and v(E) from p^E.
+constexpr uint64_t weight_lo(uint64_t pe) { return kInv179 * pe - kPrimeInv * pe; }
+constexpr uint64_t weight_hi(uint64_t pe) { return 256u * kInv179 * pe; }
+struct SumWeights {
+    uint32_t w[kHalfWords / 2][64][4];   // [word pair][lane][step]: the lane's B operand, bytes (A lo, A hi, B lo, B hi)
 };
-constexpr HalfDigits half_digits() {
-    HalfDigits t{};
-    for (int c = 0; c < kPairBytes; ++c) {
-        uint64_t va = prime_pow_of(2 * kPairBytes - c), vb = prime_pow_of(kPairBytes - c);
-        for (int j = 0; j < 4; ++j) {
-            const int32_t da = int32_t(int16_t(uint16_t(va & 0xFFFFu))), db = int32_t(int16_t(uint16_t(vb & 0xFFFFu)));
-            t.w[c][j] = (uint32_t(da) & 0xFFFFu) | (uint32_t(db) << 16);
-            va = (va - uint64_t(int64_t(da))) >> 16;
-            vb = (vb - uint64_t(int64_t(db))) >> 16;
+constexpr SumWeights sum_weights() {
+    SumWeights t{};
+    // p^(E + 4096 (3 - q)) of byte c of half A, for lane group q; half B's is 128 bytes nearer the end
+    for (int q = 0; q < 4; ++q) {
+        uint64_t pa = prime_pow_of(uint64_t(2 * kPairBytes) + 4096u * uint64_t(3 - q));
+        uint64_t pb = prime_pow_of(uint64_t(kPairBytes) + 4096u * uint64_t(3 - q));
+        for (int c = 0; c < kPairBytes; ++c) {
+            uint64_t v[4] = {weight_lo(pa), weight_hi(pa), weight_lo(pb), weight_hi(pb)};
+            const int word = c / 4, column = (word & 1) * 8;
+            for (int digit = 0; digit < 8; ++digit) {
+                uint32_t bytes = 0;
+                for (int k = 0; k < 4; ++k) {
+                    const uint64_t low = v[k] & 0xFFu;
+                    bytes |= uint32_t(low) << (8 * k);
+                    v[k] = (v[k] >> 8) + (low >= 128u ? 1u : 0u);   // the balanced digit's carry
+                }
+                t.w[word / 2][16 * q + column + digit][c % 4] = bytes;
+            }
+            pa *= kPrimeInv;
+            pb *= kPrimeInv;
         }
     }
     return t;
 }
-constexpr HalfDigits kHalfDigits = half_digits();
-// `m`: the true low byte at the segment's start in the low half, at its midpoint in the high half.
-__device__ __forceinline__ uint64_t halves_sum(const uint32_t (&w)[kFnvLaneBytes / 4], uint32_t m) {
-    int32_t s0 = 0, s1 = 0, s2 = 0, s3 = 0;
-#pragma unroll
-    for (int c = 0; c < kPairBytes; ++c) {
-        const uint32_t x = m ^ pair_byte(w[c >> 2], w[kHalfWords + (c >> 2)], c & 3);
-        const uint32_t d = pk_sub(x, m);
-        m = __umul24(x, kPrimeLow) & 0x00FF00FFu;
-        s0 = dot2(d, kHalfDigits.w[c][0], s0);
-        s1 = dot2(d, kHalfDigits.w[c][1], s1);
-        s2 = dot2(d, kHalfDigits.w[c][2], s2);
-        s3 = dot2(d, kHalfDigits.w[c][3], s3);
+__device__ const SumWeights g_sum_weights = sum_weights();
+constexpr int kWeightChunks = int(sizeof(SumWeights) / 16);
+static_assert(kWeightChunks % kFnvThreads == 0, "each lane stages whole chunks");
+// 128 times the sum of a segment's weights relative to its end: what offsetting its products' bytes takes away.
+constexpr uint64_t offset_sum() {
+    uint64_t sum = 0, pe = prime_pow_of(2 * kPairBytes);
+    for (int c = 0; c < 2 * kPairBytes; ++c, pe *= kPrimeInv) sum += weight_lo(pe) + weight_hi(pe);
+    return 128u * sum;
+}
+constexpr uint64_t kOffsetSum = offset_sum();
+// Per lane l: p^(256 (63 - l)), which takes a segment's value from its end to the end of the wave's last segment, and
+// 2^(8 (l mod 8)) p^(256 (12 - 4 (l / 16))), which does so for the lane's column and rows of the product.
+struct LanePow {
+    uint64_t v[64], col[64];
+};
+constexpr LanePow lane_pow() {
+    LanePow t{};
+    for (int l = 0; l < 64; ++l) {
+        t.v[l] = prime_pow_of(uint64_t(kFnvLaneBytes) * uint64_t(63 - l));
+        t.col[l] = prime_pow_of(uint64_t(kFnvLaneBytes) * uint64_t(12 - 4 * (l / 16))) << (8 * (l % 8));
     }
-    return digit_sum(s0, s1, s2, s3);
+    return t;
+}
+__constant__ LanePow kLanePow = lane_pow();
+
+using i32x4 = __attribute__((ext_vector_type(4))) int32_t;
+// s p^e modulo 2^64 for a signed 32-bit s: p^e as 2^32 hi + a signed low word.
+template <uint64_t kPow>
+__device__ __forceinline__ uint64_t times_pow(int32_t s) {
+    constexpr int32_t lo = int32_t(uint32_t(kPow));
+    constexpr uint32_t hi = uint32_t(kPow >> 32) + (lo < 0 ? 1u : 0u);
+    return uint64_t(int64_t(s) * int64_t(lo)) + (uint64_t(uint32_t(s) * hi) << 32);
+}
+
+// The sum over a wave's whole segments, relative to the end of the wave's last segment, spread over its lanes (their
+// values add up to it).  `w`: the step words; `m`: the true low byte at the segment's start in the low half and at its
+// midpoint in the high half.  Every lane of the wave takes part: one without a whole segment passes zeros in both,
+// whose products the correction cancels.
+__device__ __forceinline__ uint64_t wave_sum(const uint32_t (&w)[kFnvLaneBytes / 4], uint32_t m, int lane,
+                                             const u32x4* weights) {
+    const uint32_t start = m & 0xFFu;
+    i32x4 even = {0, 0, 0, 0}, odd = {0, 0, 0, 0};
+#pragma unroll
+    for (int pair = 0; pair < kHalfWords / 2; ++pair) {
+        const u32x4 b = weights[pair * 64 + lane];
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            const int k = 2 * pair + half;
+            u32x4 a;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t word = i < 2 ? w[k] : w[kHalfWords + k];
+                m = step_pair(m, (i & 1) ? word >> 8 : word);
+                a[i] = m ^ 0x80808080u;
+            }
+            const i32x4 av = __builtin_bit_cast(i32x4, a), bv = __builtin_bit_cast(i32x4, b);
+            if (half == 0) even = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, even, 0, 0, 0);
+            else odd = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bv, odd, 0, 0, 0);
+        }
+    }
+    const i32x4 s = (lane & 8) ? odd : even;
+    constexpr uint64_t p1 = prime_pow_of(kFnvLaneBytes), p2 = p1 * p1, p3 = p2 * p1;
+    const uint64_t rows = times_pow<p3>(s.x) + times_pow<p2>(s.y) + times_pow<p1>(s.z) + uint64_t(int64_t(s.w));
+    const uint64_t ends = uint64_t((m >> 16) & 0xFFu) - times_pow<p1>(int32_t(start)) + kOffsetSum;
+    return rows * kLanePow.col[lane] + ends * kLanePow.v[lane];
 }
 
 // One step of the full hash given the true low byte `l` of the state: accumulate d = (l ^ b) - l, then multiply.
@@ -174,119 +240,119 @@ __device__ __forceinline__ void step_full(uint32_t b, uint32_t& l, uint64_t& acc
     l = __umul24(x, kPrimeLow) & 0xFFu;
 }
 
-// Exclusive xor prefix of a 64-bit word: bit i of the result is the xor of bits 0..i-1.
-__device__ __forceinline__ uint64_t xor_prefix_excl(uint64_t x) {
-    x ^= x << 1;
-    x ^= x << 2;
-    x ^= x << 4;
-    x ^= x << 8;
-    x ^= x << 16;
-    x ^= x << 32;
-    return x << 1;
-}
-
-// The ballots of one level, per wave: the bits of the lanes' maps of the level (below) - the term of the lowest
-// unresolved bit j (T), of bit j + 1 for either start value a of bit j (U_a), and, in a three-bit level, of bit j + 2
-// for each start pair (a, c) of bits j, j + 1 (W_ac).
-constexpr int kMaxLevelWords = 7;   // T, U0, U1, W00, W01, W10, W11
+// ---- maps of a level ----
+// A level resolves kBits bits of the state, j .. j + kBits - 1.  A run's map of the level holds, for each of those bits and
+// each start value of the level's lower ones, the term the run xors onto the bit: bit 0 the term of bit j, bits 1-2 those
+// of bit j + 1 for start bit j = 0, 1, bits 3-6 those of bit j + 2, bits 7-14 those of bit j + 3.  The terms of bit i start
+// at 2^i - 1 and are indexed by the start bits before it as one number, the lowest bit of the state first (most
+// significant).  0 is the identity.
 template <int kBits>
-constexpr int level_words() { return kBits == 3 ? 7 : 3; }
-
-// The lanes' true start bits of one wave, as masks, from `st` (bit j in bit 0, j + 1 in bit 1, j + 2 in bit 2) at
-// the wave's first segment; `st` advances past the wave.  Each lane's term for a bit is chosen by its own true lower
-// bits, and the bit at a lane is the wave's incoming bit xor the terms of the lanes before it.
+constexpr uint32_t map_mask() { return (1u << ((1u << kBits) - 1u)) - 1u; }
 template <int kBits>
-__device__ __forceinline__ void wave_masks(const uint64_t (&wd)[kMaxLevelWords], uint32_t& st, uint64_t (&m)[3]) {
-    const uint32_t a = st & 1u, c = (st >> 1) & 1u;
-    const uint64_t sj = xor_prefix_excl(wd[0]) ^ (a ? ~0ull : 0ull);
-    const uint64_t v = (sj & wd[2]) | (~sj & wd[1]);
-    const uint64_t sc = xor_prefix_excl(v) ^ (c ? ~0ull : 0ull);
-    m[0] = sj;
-    m[1] = sc;
-    uint32_t next = (a ^ (uint32_t(__popcll(wd[0])) & 1u)) | ((c ^ (uint32_t(__popcll(v)) & 1u)) << 1);
-    if constexpr (kBits == 3) {
-        const uint32_t e = (st >> 2) & 1u;
-        const uint64_t x = (~sj & ~sc & wd[3]) | (~sj & sc & wd[4]) | (sj & ~sc & wd[5]) | (sj & sc & wd[6]);
-        m[2] = xor_prefix_excl(x) ^ (e ? ~0ull : 0ull);
-        next |= (e ^ (uint32_t(__popcll(x)) & 1u)) << 2;
-    }
-    st = next;
+constexpr uint32_t state_mask() { return (1u << kBits) - 1u; }
+
+// A run's map from its machines' end states: e[m] ended the machine started from the true lower bits, m in the level's
+// lowest kBits - 2 bits and zeros above.  The top bit's terms for a set start bit below it follow from that bit's own term,
+// the parity of that bit over the run's bytes (`par`, the xor of the bytes) and the run's length (`odd`).
+template <int kJ, int kBits>
+__device__ __forceinline__ uint32_t map_of(const uint32_t (&e)[1 << (kBits - 2)], uint32_t par, uint32_t odd) {
+    const uint32_t flip = ((par >> (kJ + kBits - 2)) & 1u) ^ odd;
+    uint32_t m = 0;
+#pragma unroll
+    for (int i = 0; i < kBits; ++i)
+#pragma unroll
+        for (int at = 0; at < (1 << i); ++at) {   // the start bits before bit i, the first most significant
+            int machine = 0;
+#pragma unroll
+            for (int k = 0; k < i && k < kBits - 2; ++k) machine |= ((at >> (i - 1 - k)) & 1) << k;
+            uint32_t term = (e[machine] >> (kJ + i)) & 1u;
+            if (i == kBits - 1 && (at & 1)) term ^= ((e[machine] >> (kJ + kBits - 2)) & 1u) ^ flip;
+            m |= term << ((1 << i) - 1 + at);
+        }
+    return m;
 }
 
-// The first level only needs bits 0..2 of the state, which follow l' = ((l ^ b) * 3) mod 8 (179 = 3 mod 8): four
-// such machines share one register, one per byte (a 3-bit state times 3 stays below 2^8, so nothing carries across
-// bytes; the product's bits above 2 are masked by the next step).
-__device__ __forceinline__ uint32_t step_low3(uint32_t x, uint32_t b4) {
-    const uint32_t y = (x ^ b4) & 0x07070707u;
-    return y + (y << 1);
-}
-
-// A run's map of a level from its machines' end states.  Three-bit level for bits j..j+2: e0 and e1 ended the machines
-// started from the true lower bits with bit j = 0 and 1 (bits j + 1, j + 2 = 0); two-bit level for bits j, j + 1: e
-// ended the one machine started with both 0.  The bits the machines do not give follow from the term of the bit below,
-// the parity of that bit over the run's bytes (bit i of `par`, the xor of the bytes) and the run's length (`odd`).
-template <int j>
-__device__ __forceinline__ uint32_t map3_of(uint32_t e0, uint32_t e1, uint32_t par, uint32_t odd) {
-    const uint32_t t = (e0 >> j) & 1u, v0 = (e0 >> (j + 1)) & 1u, v1 = (e1 >> (j + 1)) & 1u;
-    const uint32_t w00 = (e0 >> (j + 2)) & 1u, w10 = (e1 >> (j + 2)) & 1u, q = ((par >> (j + 1)) & 1u) ^ odd;
-    return t | (v0 << 1) | (v1 << 2) | (w00 << 3) | ((w00 ^ v0 ^ q) << 4) | (w10 << 5) | ((w10 ^ v1 ^ q) << 6);
-}
-template <int j>
-__device__ __forceinline__ uint32_t map2_of(uint32_t e, uint32_t par, uint32_t odd) {
-    const uint32_t t = (e >> j) & 1u, v0 = (e >> (j + 1)) & 1u;
-    return t | (v0 << 1) | ((v0 ^ t ^ ((par >> j) & 1u) ^ odd) << 2);
-}
-
-// The same maps of a partial or unaligned segment (whole segments run from registers, below), a byte at a time from
-// memory; `low` holds the true bits below j at the segment's start.
-template <int j>
-__device__ __forceinline__ uint32_t map3_bytes(const uint8_t* p, uint64_t n, uint32_t low) {
-    uint32_t x = low | ((low | (1u << j)) << 16), par = 0;
-    for (uint64_t i = 0; i < n; ++i) {
+// The same map of a partial or unaligned segment (whole segments run from registers, below), a byte at a time from
+// memory; `low` holds the true bits below kJ at the segment's start.
+template <int kJ, int kBits>
+__device__ __forceinline__ uint32_t map_bytes(const uint8_t* p, uint32_t n, uint32_t low) {
+    uint32_t e[1 << (kBits - 2)], par = 0;
+#pragma unroll
+    for (uint32_t m = 0; m < (1u << (kBits - 2)); ++m) e[m] = low | (m << kJ);
+    for (uint32_t i = 0; i < n; ++i) {
         const uint32_t b = p[i];
         par ^= b;
-        x = step_pair(x, b * 0x10001u);
+#pragma unroll
+        for (uint32_t& x : e) x = __umul24((x ^ b) & 0xFFu, kPrimeLow);
     }
-    return map3_of<j>(x & 0xFFFFu, x >> 16, par, uint32_t(n & 1u));
-}
-template <int j>
-__device__ __forceinline__ uint32_t map2_bytes(const uint8_t* p, uint64_t n, uint32_t low) {
-    uint32_t x = low, par = 0;
-    for (uint64_t i = 0; i < n; ++i) {
-        const uint32_t b = p[i];
-        par ^= b;
-        x = step_pair(x, b * 0x10001u);
-    }
-    return map2_of<j>(x, par, uint32_t(n & 1u));
+    return map_of<kJ, kBits>(e, par, n & 1u);
 }
 
-// A workgroup's map of a level's state: (a, c, e) = (bit j, j + 1, j + 2) at its first segment goes to
-// (a ^ t, c ^ v_a, e ^ w_ac) at the next workgroup's first segment; the map is a byte (bit 0 t, bits 1-2 v_0 v_1,
-// bits 3-6 w_00 w_01 w_10 w_11; a two-bit level has no e and no w), 0 being the identity.  Maps compose as
-// (g after f): t = t_f ^ t_g, v_a = v_a(f) ^ v_(a ^ t_f)(g), w_ac = w_ac(f) ^ w_(a ^ t_f, c ^ v_a(f))(g).
-__device__ __forceinline__ uint32_t map_v(uint32_t m, uint32_t a) { return (m >> (1u + a)) & 1u; }
-__device__ __forceinline__ uint32_t map_w(uint32_t m, uint32_t a, uint32_t c) { return (m >> (3u + 2u * a + c)) & 1u; }
-template <int kBits>
-__device__ __forceinline__ uint32_t compose(uint32_t g, uint32_t f) {
-    const uint32_t tf = f & 1u;
-    uint32_t r = tf ^ (g & 1u);
-#pragma unroll
-    for (uint32_t a = 0; a < 2; ++a) r |= (map_v(f, a) ^ map_v(g, a ^ tf)) << (1u + a);
-    if constexpr (kBits == 3) {
-#pragma unroll
-        for (uint32_t a = 0; a < 2; ++a)
-#pragma unroll
-            for (uint32_t c = 0; c < 2; ++c)
-                r |= (map_w(f, a, c) ^ map_w(g, a ^ tf, c ^ map_v(f, a))) << (3u + 2u * a + c);
-    }
-    return r;
-}
+// The state after a map.
 template <int kBits>
 __device__ __forceinline__ uint32_t apply(uint32_t m, uint32_t st) {
-    const uint32_t a = st & 1u, c = (st >> 1) & 1u;
-    uint32_t r = (a ^ (m & 1u)) | ((c ^ map_v(m, a)) << 1);
-    if constexpr (kBits == 3) r |= (((st >> 2) & 1u) ^ map_w(m, a, c)) << 2;
+    uint32_t out = st, at = 0;
+#pragma unroll
+    for (int i = 0; i < kBits; ++i) {
+        out ^= ((m >> ((1u << i) - 1u + at)) & 1u) << i;
+        at = 2u * at + ((st >> i) & 1u);
+    }
+    return out;
+}
+
+// g after f.  `at` are the start bits before bit kBit in f, `gat` what they have become where g starts; the top bit's
+// terms are taken two at a time, g's pair swapped where f flips the bit below.
+template <int kBits, int kBit = 0>
+__device__ __forceinline__ uint32_t compose(uint32_t g, uint32_t f, uint32_t at = 0, uint32_t gat = 0) {
+    constexpr uint32_t base = (1u << kBit) - 1u, next = (2u << kBit) - 1u;
+    const uint32_t t = (f >> (base + at)) & 1u;
+    uint32_t r = (t ^ ((g >> (base + gat)) & 1u)) << (base + at);
+    if constexpr (kBit + 2 == kBits) {
+        const uint32_t pair = (g >> (next + 2u * gat)) & 3u, swapped = (pair >> 1) | ((pair & 1u) << 1);
+        r |= (((f >> (next + 2u * at)) & 3u) ^ (t ? swapped : pair)) << (next + 2u * at);
+    } else {
+        r |= compose<kBits, kBit + 1>(g, f, 2u * at, 2u * gat + t) |
+             compose<kBits, kBit + 1>(g, f, 2u * at + 1u, 2u * gat + (t ^ 1u));
+    }
     return r;
+}
+
+// The maps of a wave's lanes, lane after lane.  A bit at a lane is the wave's start bit xor the parity of the terms of the
+// lanes before it, and each lane's term is picked by its own true lower bits: a ballot, a count of the lower lanes (mbcnt)
+// and a shift per term, on the vector units (as 64-bit scalar xor prefixes, 12 dependent operations each, the same took
+// twice the instructions on the path that every later workgroup waits for).
+__device__ __forceinline__ uint32_t lower_parity(uint64_t mask) {
+    return __builtin_amdgcn_mbcnt_hi(uint32_t(mask >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(mask), 0u)) & 1u;
+}
+__device__ __forceinline__ uint32_t parity(uint64_t mask) { return uint32_t(__popcll(mask)) & 1u; }
+__device__ __forceinline__ uint64_t ballot_bit(uint32_t v) { return __ballot((v & 1u) != 0u); }
+// The wave's map.  `at` are the wave's start bits before bit kBit, `lane_at` what they are at the lane.
+template <int kBits, int kBit = 0>
+__device__ __forceinline__ uint32_t wave_map(uint32_t lane_map, uint32_t at = 0, uint32_t lane_at = 0) {
+    constexpr uint32_t base = (1u << kBit) - 1u;
+    const uint64_t t = ballot_bit(lane_map >> (base + lane_at));
+    uint32_t m = parity(t) << (base + at);
+    if constexpr (kBit + 1 < kBits) {
+        const uint32_t p = lower_parity(t);
+        m |= wave_map<kBits, kBit + 1>(lane_map, 2u * at, 2u * lane_at + p) |
+             wave_map<kBits, kBit + 1>(lane_map, 2u * at + 1u, 2u * lane_at + (p ^ 1u));
+    }
+    return m;
+}
+// Through the wave from its start state `st`: its end state, and this lane's start state in `at_lane`.
+template <int kBits>
+__device__ __forceinline__ uint32_t wave_apply(uint32_t lane_map, uint32_t st, uint32_t& at_lane) {
+    uint32_t end = st, at = 0;
+    at_lane = 0;
+#pragma unroll
+    for (int i = 0; i < kBits; ++i) {
+        const uint64_t t = ballot_bit(lane_map >> ((1u << i) - 1u + at));
+        const uint32_t bit = lower_parity(t) ^ ((st >> i) & 1u);
+        end ^= parity(t) << i;
+        at_lane |= bit << i;
+        at = 2u * at + bit;
+    }
+    return end;
 }
 
 // The state the hash starts from: the launch's seed, or the running hash at `seed_dev` when the input continues an
@@ -316,10 +382,19 @@ __device__ __forceinline__ uint64_t segment_sum(const uint8_t* p, uint64_t n, ui
 // earlier pieces left there, so a chain reports a fault of any of its pieces.  With `verdict`, also 1 there when h
 // equals `expected` and the launch has no fault, else 0: a later kernel on the stream can act on the check without a
 // host round trip.
-__global__ void fnv_finish_kernel(const uint64_t* acc, uint64_t seed, const uint64_t* seed_dev, uint64_t n, uint64_t* out,
+__global__ void fnv_finish_kernel(const uint32_t* ctl, uint64_t seed, const uint64_t* seed_dev, uint64_t n, uint64_t* out,
                                   uint32_t* fault_out, bool sticky, uint64_t expected, uint32_t* verdict,
-                                  const uint32_t* fault, const uint8_t* tail, uint32_t tail_len) {
-    uint64_t h = start_state(seed, seed_dev) * pow_prime(n) + (acc ? acc[0] : 0u);
+                                  const uint8_t* tail, uint32_t tail_len) {
+    // the whole segments' sums are relative to the end of the last workgroup's 64 KiB
+    uint64_t h = start_state(seed, seed_dev) * pow_prime(n);
+    if (ctl) {
+        const uint64_t* acc = reinterpret_cast<const uint64_t*>(ctl + 2);
+        const uint64_t past = (kFnvGroupBytes - n % kFnvGroupBytes) % kFnvGroupBytes;
+        uint64_t back = 1, b = kPrimeInv;
+        for (uint64_t e = past; e; e >>= 1, b *= b)
+            if (e & 1) back *= b;
+        h += acc[0] * back + acc[1];
+    }
     // the mapped hash leaves the payload's last partial lane segment (under 256 bytes, whole 16-byte chunks at a 16-byte
     // aligned address) to this thread: its chunks are loaded at once, then hashed a byte at a time from registers
     // (a loop of byte loads took 14 us, each load waiting on the one before)
@@ -337,27 +412,26 @@ __global__ void fnv_finish_kernel(const uint64_t* acc, uint64_t seed, const uint
                 if (uint32_t(k) * 16u + uint32_t(b) < tail_len) h = (h ^ ((word[b / 4] >> (8 * (b % 4))) & 0xFFu)) * kFnvPrime;
         }
     }
-    const uint32_t bad = fault ? fault[0] : 0u;   // kFaultWait and / or kFaultCarry
+    const uint32_t bad = ctl ? ctl[1] : 0u;   // kFaultWait and / or kFaultCarry
     out[0] = h;
     if (fault_out) fault_out[0] = sticky ? (fault_out[0] | bad) : bad;
     if (verdict) verdict[0] = h == expected && !bad ? 1u : 0u;
 }
 
 // ---- the one-pass hash ---------------------------------------------------------------------------------------------
-// One kernel reads the input once: each lane keeps its 256-byte segment in registers through the three levels of the
-// low byte and the Horner sums.  A level's workgroup start state comes from a decoupled look-back rather than a scan
-// kernel: workgroups take their index from a ticket counter in the order they start, publish their map of the level's
-// state as soon as they have it and their end state once they know their start, and a workgroup finds its start by
-// reading the words of the 64 workgroups before it at once and composing maps back to the nearest end state.  A
-// workgroup waits only on lower tickets, held by workgroups that are running or done, so every wait ends; each wait is
-// also bounded (kSpinLimit reads), after which the launch records a fault that fails the verdict and the workgroup
-// publishes an end state anyway, so no other workgroup waits on it.
+// One kernel reads the input once: each lane keeps its 256-byte segment in registers through the levels of the low byte
+// and the sums.  A level's workgroup start state comes from a decoupled look-back rather than a scan kernel: workgroups
+// take their index from a ticket counter in the order they start, publish their map of the level's state as soon as they
+// have it and their end state once they know their start, and a workgroup finds its start by reading the words of the 64
+// workgroups before it at once and composing maps back to the nearest end state.  A workgroup waits only on lower tickets,
+// held by workgroups that are running or done, so every wait ends; each wait is also bounded (kSpinLimit reads), after
+// which the launch records a fault that fails the verdict and the workgroup publishes an end state anyway, so no other
+// workgroup waits on it.
 // The lane within its wave, from the exec-independent lane count (two VALU operations): used where keeping threadIdx.x
 // live across the kernel would spill it and reload it from scratch, a memory round trip each time.
 __device__ __forceinline__ int lane_id() { return int(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u))); }
-constexpr uint32_t kHasMap = 1u << 8, kHasState = 1u << 9;   // a status word: 0, kHasMap | map, kHasState | state
 // Sleeps of 64 x 64 cycles before a look-back's first read of its window (the mapped kernel's last level writes its
-// gathered payload instead): 3.3 GB hashed in 1.77 ms with two, 1.79 ms with none
+// gathered payload instead): 3.3 GB hashed in 1.36 ms with two, 1.38 with one or three
 constexpr int kFirstSleeps = 2, kFirstSleepsMapped = 0;
 constexpr uint32_t kSpinLimit = 1u << 16;   // reads of one window, about 0.2 s (sc_fnv1a64_set_spin_limit)
 // A bound the host sets only to test failure handling: every look-back of a workgroup after the first runs out at
@@ -370,212 +444,221 @@ constexpr uint32_t kFaultWait = SC_FNV_FAULT_WAIT, kFaultCarry = SC_FNV_FAULT_CA
 __device__ __forceinline__ void flag_fault(uint32_t* fault, uint32_t v) {
     __hip_atomic_fetch_or(fault, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ void publish(uint32_t* word, uint32_t v) {
-    __hip_atomic_store(word, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ void publish(uint32_t* status, uint32_t v) {
+    __hip_atomic_store(status, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ uint32_t peek(uint32_t* word) {
-    return __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+__device__ __forceinline__ uint32_t peek(const uint32_t* status) {
+    return __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Workgroup g's start state at one level, run by one whole wave (the result is wave-uniform); publishes g's map
-// before the look-back and its end state after.  `init` is the state before workgroup 0.  Lane l reads the word of
-// workgroup top - l.  The maps of lanes 0..l compose in one inclusive scan across the wave (six shuffle steps), so
-// resolving a window costs the same wherever its nearest end state lies.
-template <int kBits>
-__device__ __forceinline__ uint32_t look_back(uint32_t* status, uint64_t g, uint32_t map, uint32_t init, uint32_t* fault,
-                                              uint32_t spin_limit, int first_sleeps) {
+// The one-pass kernel's arguments.  They are read where they are needed, through the argument segment with scalar loads
+// (kernel_args: a pointer that is new to the compiler each time): held in scalar registers across the kernel they pushed
+// its wave masks out of them (70-95 spilled scalars).
+template <int v>
+using Int = std::integral_constant<int, v>;
+struct OnepassArgs {
+    const uint8_t* data;        // the input (16-byte aligned: `aligned`), or null with `map`
+    uint64_t n;                 // bytes hashed in the kernel
+    uint64_t seed;
+    const uint64_t* seed_dev;
+    uint32_t* ctl;              // [0] the ticket counter, [1] the fault word, [2..3], [4..5] the sums of whole and of partial segments
+    uint32_t* status;           // [workgroup][level], kStatusWords each
+    HashMapArgs map;
+    FnvCarries carries;
+    uint64_t carry_count;
+    uint32_t groups;            // workgroups' worth of input (64 KiB each)
+    uint32_t spin_limit;
+    uint32_t aligned;
+};
+using ConstArgs = const __attribute__((address_space(4))) OnepassArgs;
+__device__ __forceinline__ ConstArgs* kernel_args() {
+    ConstArgs* p = (ConstArgs*) __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
+}
+// The low byte the hash starts from.
+__device__ __forceinline__ uint32_t start_byte() {
+    ConstArgs* a = kernel_args();
+    return uint32_t(start_state(a->seed, a->seed_dev)) & 0xFFu;
+}
+
+// A workgroup's status word of one level: 0, kHasMap | map or kHasState | state.
+constexpr uint32_t kHasMap = 1u << 16, kHasState = 1u << 17;
+// The levels of a hash that looks back: two of four bits.  Each costs a wait of 6-7 us (see fnv_onepass_kernel), more than
+// the machines a third level saves (13.5 vector operations per two bytes with three levels of 3, 3 and 2 bits, 17 with two):
+// 3.3 GB in 1.36 against 1.41 ms, the 128K capture and hash in 1.76 against 1.89 ms.  A check given carries never waits
+// and takes the three levels: 0.87 against 1.02 ms.
+constexpr uint32_t kStatusWords = 2;
+
+// Workgroup g's start state at one level, run by one whole wave (the result is wave-uniform); the caller has published
+// g's map, and its end state is published after.  Lane l reads the status word of workgroup top - 64 + l; before workgroup
+// 0 stands the start state.  The maps after the nearest end state compose like those of a wave's lanes, so resolving a
+// window costs the same wherever that state lies.  Reading 128 or 256 words at once measured slower (1.66 and 1.87 ms for
+// 3.3 GB against 1.60: every read of a line that other XCDs write costs them all).
+template <int kLevel, int kJ, int kBits>
+__device__ __forceinline__ uint32_t look_back(uint32_t g, uint32_t map, int first_sleeps) {
     const int lane = lane_id();
-    if (g == 0) {
-        if (lane == 0) publish(status, kHasState | apply<kBits>(map, init));
-        return init;
-    }
-    if (spin_limit == kForceFault) {   // the failure-handling tests' forced fault (never set otherwise)
-        if (lane == 0) {
-            flag_fault(fault, kFaultWait);
-            publish(status + g, kHasState | apply<kBits>(map, 0u));
-        }
-        return 0u;
-    }
-    // the caller has published g's map.  The workgroups just before g publish theirs a few microseconds after g on
-    // average (their work varies with what shares their SIMDs), so a read right away would mostly find the window
-    // incomplete and cost a round trip and a sleep anyway
+    uint32_t* const status = kernel_args()->status + kLevel;
+    const auto settle = [&](uint32_t st) {
+        if (lane == 0) publish(status + g * kStatusWords, kHasState | apply<kBits>(map, st));
+        return st;
+    };
+    const auto fault = [&] {   // successors still get an end state
+        if (lane == 0) flag_fault(kernel_args()->ctl + 1, kFaultWait);
+        return settle(0u);
+    };
+    const uint32_t init = g < 64u ? (start_byte() >> kJ) & state_mask<kBits>() : 0u;
+    if (g == 0) return settle(init);
+    const uint32_t spin_limit = kernel_args()->spin_limit;
+    if (spin_limit == kForceFault) return fault();   // the failure-handling tests' forced fault (never set otherwise)
+    // the workgroups just before g publish their maps about 2 us after g on average (their work varies with what shares
+    // their SIMDs), so a read right away would mostly find the window incomplete and cost a round trip and a sleep anyway
     for (int i = 0; i < first_sleeps; ++i) __builtin_amdgcn_s_sleep(64);
-    uint32_t acc = 0;                  // the maps of the workgroups from above the window up to g, composed
-    int64_t top = int64_t(g) - 1;      // the window is workgroups top, top - 1, ...; before workgroup 0 stands `init`
+    uint32_t acc = 0;   // the maps of the workgroups from `top` up to g, composed
     uint32_t spins = 0;
-    for (;;) {
-        const int64_t h = top - lane;
-        const uint32_t word = h >= 0 ? peek(status + h) : (kHasState | init);
-        const uint64_t have_state = __ballot((word & kHasState) != 0u);
-        const uint64_t ready = __ballot((word & (kHasMap | kHasState)) != 0u);
-        const int first = have_state ? __builtin_ctzll(have_state) : 64;   // the lane of the nearest end state
-        const uint64_t need = first == 64 ? ~0ull : (1ull << first) - 1ull;
-        if ((ready & need) != need) {   // a workgroup between g and that end state has not published its map yet
-            if (++spins > spin_limit) {   // never in a correct launch; successors still get an end state
-                if (lane == 0) {
-                    flag_fault(fault, kFaultWait);
-                    publish(status + g, kHasState | apply<kBits>(map, 0u));
-                }
-                return 0u;
-            }
-            // a long sleep (64 x 64 cycles, about 1.7 us) leaves the SIMD's issue slots to the other waves' level work:
-            // sleeps of 16 or 32 between reads measured slower (1.77-1.78 against 1.76 ms for 3.3 GB; the fused
-            // capture 2.42-2.47 against 2.37 ms), and so did 1 in the earlier form of the levels
+    for (int32_t top = int32_t(g);;) {
+        const int32_t h = top - 64 + lane;
+        const uint32_t word = h >= 0 ? peek(status + uint32_t(h) * kStatusWords) : (kHasState | init);
+        const uint64_t have_state = __ballot((word & kHasState) != 0u), ready = __ballot(word != 0u);
+        const int at = have_state ? 63 - __builtin_clzll(have_state) : -1;   // the lane of the nearest end state
+        const uint64_t need = at == 63 ? 0u : ~0ull << (at + 1);
+        if ((ready & need) != need) {   // a workgroup between that end state and g has not published its map yet
+            if (++spins > spin_limit) return fault();   // never in a correct launch
+            // a long sleep (64 x 64 cycles, about 1.7 us) leaves the SIMD's issue slots to the other waves' level work and
+            // the status lines to their writers: sleeps of 8-32 measured alike for the plain hash and slower for the
+            // fused one
             __builtin_amdgcn_s_sleep(64);
             continue;
         }
-        // x_l = map_0 o map_1 o ... o map_l (map_l applied first); the lanes from `first` on are not used
-        uint32_t x = word & 0xFFu;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const uint32_t lower = uint32_t(__shfl_up(int(x), d));
-            if (lane >= d) x = compose<kBits>(lower, x);
+        const uint32_t after = lane > at ? word & map_mask<kBits>() : 0u;   // the maps after that end state
+        if (at >= 0) {
+            uint32_t unused;
+            const uint32_t st = uint32_t(__builtin_amdgcn_readlane(int(word), at)) & state_mask<kBits>();
+            return settle(apply<kBits>(acc, wave_apply<kBits>(after, st, unused)));
         }
-        if (first < 64) {
-            uint32_t st = uint32_t(__builtin_amdgcn_readlane(int(word), first)) & 0xFFu;
-            if (first > 0) st = apply<kBits>(uint32_t(__builtin_amdgcn_readlane(int(x), first - 1)), st);
-            st = apply<kBits>(acc, st);
-            if (lane == 0) publish(status + g, kHasState | apply<kBits>(map, st));
-            return st;
-        }
-        acc = compose<kBits>(acc, uint32_t(__builtin_amdgcn_readlane(int(x), 63)));   // all maps: read the window before
+        acc = compose<kBits>(acc, wave_map<kBits>(after));   // all maps: read the window before
         top -= 64;
         spins = 0;
     }
 }
 
+// (p^65536)^k as a product of one entry per byte of k: what a workgroup's sum is worth k whole 64 KiB before the last.
+struct GroupPow {
+    uint64_t v[4][256];
+};
+constexpr GroupPow group_pows() {
+    GroupPow t{};
+    uint64_t step = prime_pow_of(uint64_t(kFnvGroupBytes));
+    for (int i = 0; i < 4; ++i) {
+        uint64_t x = 1;
+        for (int k = 0; k < 256; ++k, x *= step) t.v[i][k] = x;
+        step = x;
+    }
+    return t;
+}
+__constant__ GroupPow kGroupPow = group_pows();
+__device__ __forceinline__ uint64_t group_pow(int byte, uint32_t k) { return kGroupPow.v[byte][(k >> (8 * byte)) & 255u]; }
+
 struct LevelLds {
-    uint64_t bw[kFnvThreads / 64][kMaxLevelWords];
-    uint32_t map[kFnvThreads / 64];
-    uint32_t state;
+    uint32_t map[3][kFnvThreads / 64];   // per level, so that a level's maps are not rewritten while they are read
+    uint32_t state, ticket;
+    uint64_t sum[kFnvThreads / 64], part[kFnvThreads / 64];   // the waves' sums of whole and of partial segments
 };
 
-__device__ __forceinline__ uint64_t uniform64(uint64_t v) {
-    return uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(v))))) |
-           (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(v >> 32))))) << 32);
-}
-
-// One level (bits j .. j + kBits - 1) once every lane has its map of the level (`lane_map`, the identity 0 for a lane
-// past the input): ballots the maps, forms and publishes the workgroup's map, runs `during` in every wave (work that
-// does not need the level's result, done while the look-back waits), looks back for the workgroup's start state after
-// `first_sleeps` sleeps of 64 x 64 cycles, and returns this lane's start bits of the level (bit 0 upward).
-template <int kBits, typename During>
-__device__ __forceinline__ uint32_t resolve_level(int wave, uint32_t lane_map, uint64_t g, uint32_t* status, uint32_t init,
-                                                  uint32_t* fault, uint32_t spin_limit, LevelLds& L, int first_sleeps,
-                                                  During during, int j, const uint8_t* carry_in, uint64_t carry_count,
-                                                  uint32_t& end_bits) {
-    uint64_t bw[kMaxLevelWords] = {};
-#pragma unroll
-    for (int i = 0; i < level_words<kBits>(); ++i) bw[i] = __ballot((lane_map >> i) & 1u);
-    uint32_t wmap = 0;
-#pragma unroll
-    for (uint32_t in = 0; in < (1u << (kBits - 1)); ++in) {
-        const uint32_t a = in & 1u, c = (in >> 1) & 1u;
-        uint32_t st = in;
-        uint64_t m[3];
-        wave_masks<kBits>(bw, st, m);
-        if (in == 0) wmap |= st & 1u;
-        if (c == 0) wmap |= ((st >> 1) & 1u) << (1 + a);
-        if constexpr (kBits == 3) wmap |= ((st >> 2) & 1u) << (3 + 2 * a + c);
-    }
+// One level, once every lane has its map of the level (`lane_map`, the identity 0 for a lane past the input): forms and
+// publishes the workgroup's map, runs `during` in every wave (work that does not need the level's result, done while the
+// look-back waits), looks back for the workgroup's start state after `first_sleeps` sleeps of 64 x 64 cycles, and returns
+// this lane's start bits of the level (bit 0 upward); `end_bits` gathers the workgroup's end state.  Given carries
+// (`before` is the one before the workgroup, its start state), every wave has the start state at once.
+template <bool kCarried, int kLevel, int kJ, int kBits, typename During>
+__device__ __forceinline__ uint32_t resolve_level(int wave, uint32_t lane_map, uint32_t g, LevelLds& L, int first_sleeps,
+                                                  During during, uint32_t before, uint32_t& end_bits) {
     const int lane = lane_id();
-    if (lane == 0) {
-#pragma unroll
-        for (int i = 0; i < level_words<kBits>(); ++i) L.bw[wave][i] = bw[i];
-        L.map[wave] = wmap;
-    }
+    const uint32_t own = wave_map<kBits>(lane_map);
+    if (lane == 0) L.map[kLevel][wave] = own;
     __syncthreads();
-    uint32_t sum = L.map[0];
-    if (wave == 0) {
-        for (int k = 1; k < kFnvThreads / 64; ++k) sum = compose<kBits>(L.map[k], sum);
-        sum = __builtin_amdgcn_readfirstlane(sum);
-        if (lane == 0 && g > 0 && !carry_in) publish(status + g, kHasMap | sum);
-    }
-    during();
-    if (wave == 0) {
-        constexpr uint32_t kMask = (1u << kBits) - 1u;
-        uint32_t st;
-        if (carry_in) {   // the start is the carry before the workgroup, checked by the one after it
-            st = g == 0 ? init : (uint32_t(carry_in[g - 1]) >> j) & kMask;
-            if (g < carry_count && apply<kBits>(sum, st) != ((uint32_t(carry_in[g]) >> j) & kMask) && lane == 0)
-                flag_fault(fault, kFaultCarry);
-        } else {
-            st = look_back<kBits>(status, g, sum, init, fault, spin_limit, first_sleeps);
+    // the waves' maps, lane k holding wave k's, compose as a wave's lanes do
+    const uint32_t waves = lane < kFnvThreads / 64 ? L.map[kLevel][lane] : 0u;
+    uint32_t st;
+    if constexpr (kCarried) {
+        during();
+        st = (before >> kJ) & state_mask<kBits>();
+    } else {
+        uint32_t sum = 0;
+        if (wave == 0) {
+            sum = wave_map<kBits>(waves);
+            if (lane == 0 && g > 0) publish(kernel_args()->status + g * kStatusWords + kLevel, kHasMap | sum);
         }
-        if (lane == 0) L.state = st;
-        end_bits |= apply<kBits>(sum, st) << j;
+        during();
+        if (wave == 0) {
+            st = look_back<kLevel, kJ, kBits>(g, sum, first_sleeps);
+            if (lane == 0) L.state = st;
+        }
+        __syncthreads();
+        st = __builtin_amdgcn_readfirstlane(L.state);
     }
-    __syncthreads();
-    uint32_t st = __builtin_amdgcn_readfirstlane(L.state);
-    uint64_t m[3] = {0, 0, 0};
-#pragma unroll
-    for (int k = 0; k < kFnvThreads / 64; ++k) {
-        if (k > wave) break;
-        uint64_t wd[kMaxLevelWords] = {};
-#pragma unroll
-        for (int i = 0; i < level_words<kBits>(); ++i) wd[i] = uniform64(L.bw[k][i]);
-        wave_masks<kBits>(wd, st, m);
-    }
-    uint32_t bits = 0;
-#pragma unroll
-    for (int i = 0; i < kBits; ++i) bits |= (uint32_t(m[i] >> lane) & 1u) << i;
-    __syncthreads();   // the next level rewrites L
+    uint32_t at_wave, bits;
+    end_bits |= wave_apply<kBits>(waves, st, at_wave) << kJ;
+    (void) wave_apply<kBits>(lane_map, uint32_t(__builtin_amdgcn_readlane(int(at_wave), wave)), bits);
     return bits;
 }
 
 // The levels of a whole segment held in registers, run as its two halves of kPairBytes bytes side by side (half A the
-// first, half B the second): each returns half A's map of the level in its low 16 bits and half B's above.  `par` holds
-// the xor of half A's bytes in byte 0 and of half B's in byte 2, `low` the true bits below the level at half A's start
-// in byte 0 and at half B's in byte 2.
+// first, half B the second): half A's map of the level in the low 16 bits and half B's above.  `w` holds the step words
+// (pair_words), `par` the xor of half A's bytes in byte 0 and of half B's in byte 2, `low` the true bits
+// below the level at half A's start in byte 0 and at half B's in byte 2.
 __device__ __forceinline__ uint32_t half_parities(const uint32_t (&w)[kFnvLaneBytes / 4]) {
-    uint32_t a = 0, b = 0;
+    uint32_t z = 0;
 #pragma unroll
-    for (int k = 0; k < kHalfWords; ++k) {
-        a ^= w[k];
-        b ^= w[kHalfWords + k];
-    }
-    a ^= a >> 16;
-    a ^= a >> 8;
-    b ^= b >> 16;
-    b ^= b >> 8;
-    return (a & 0xFFu) | ((b & 0xFFu) << 16);
+    for (int k = 0; k < kFnvLaneBytes / 4; ++k) z ^= w[k];
+    return (z ^ (z >> 8)) & 0x00FF00FFu;
 }
-// Byte k of `a` in bytes 0 and 1, byte k of `b` in bytes 2 and 3.
-__device__ __forceinline__ uint32_t pair_byte2(uint32_t a, uint32_t b, int k) {
-    return __builtin_amdgcn_perm(b, a, uint32_t(k) | (uint32_t(k) << 8) | (uint32_t(4 + k) << 16) | (uint32_t(4 + k) << 24));
-}
-// Bits 0-2: four 3-bit machines, half A's started from bit 0 = 0 and 1 in bytes 0 and 1, half B's in bytes 2 and 3.
-__device__ __forceinline__ uint32_t level1_maps(const uint32_t (&w)[kFnvLaneBytes / 4], uint32_t par) {
-    uint32_t x = 0x01000100u;
+template <int kJ, int kBits>
+__device__ __forceinline__ uint32_t level_maps(const uint32_t (&w)[kFnvLaneBytes / 4], uint32_t low, uint32_t par) {
+    constexpr int kMachines = 1 << (kBits - 2);
+    uint32_t a[kMachines], b[kMachines];
+    if constexpr (kJ == 0) {
+        // the lowest bits follow l' = 3 (l ^ b) mod 2^kBits (179 = 3 mod 16): a machine takes one byte of a register
+        // (three times a 4-bit state stays below 2^8, and the next step masks what is above the state), half A's from
+        // bit 0 = 0 and 1 in bytes 0 and 1, half B's in bytes 2 and 3, register m from m in the bits above
+        static_assert(kBits == 3 || kBits == 4, "the machines' products stay in their bytes");
+        constexpr uint32_t kMask = state_mask<kBits>() * 0x01010101u;
+        uint32_t x[kMachines / 2];
 #pragma unroll
-    for (int k = 0; k < kHalfWords; ++k)
+        for (uint32_t m = 0; m < kMachines / 2; ++m) x[m] = 2u * m * 0x01010101u + 0x01000100u;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) x = step_low3(x, pair_byte2(w[k], w[kHalfWords + k], i));
-    return map3_of<0>(x & 0xFFu, (x >> 8) & 0xFFu, par, 0u) |
-           (map3_of<0>((x >> 16) & 0xFFu, x >> 24, par >> 16, 0u) << 16);
-}
-// Bits 3-5: half A's machines in byte 0 of r0 (start bit 3 = 0) and r1 (= 1), half B's in their byte 2.
-__device__ __forceinline__ uint32_t level2_maps(const uint32_t (&w)[kFnvLaneBytes / 4], uint32_t low, uint32_t par) {
-    uint32_t r0 = low, r1 = low | 0x00080008u;
+        for (int k = 0; k < kHalfWords; ++k)
 #pragma unroll
-    for (int k = 0; k < kHalfWords; ++k)
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t word = i < 2 ? w[k] : w[kHalfWords + k];
+                const uint32_t b4 = __builtin_amdgcn_perm(word, word, (i & 1) ? 0x03030101u : 0x02020000u);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t bb = pair_byte(w[k], w[kHalfWords + k], i);
-            r0 = step_pair(r0, bb);
-            r1 = step_pair(r1, bb);
+                for (uint32_t& m : x) {
+                    const uint32_t y = (m ^ b4) & kMask;
+                    m = y + (y << 1);
+                }
+            }
+#pragma unroll
+        for (int m = 0; m < kMachines; ++m) {
+            a[m] = x[m >> 1] >> (8 * (m & 1));
+            b[m] = x[m >> 1] >> (16 + 8 * (m & 1));
         }
-    return map3_of<3>(r0 & 0xFFu, r1 & 0xFFu, par, 0u) |
-           (map3_of<3>((r0 >> 16) & 0xFFu, (r1 >> 16) & 0xFFu, par >> 16, 0u) << 16);
-}
-// Bits 6-7: one machine per half, half A's in byte 0, half B's in byte 2.
-__device__ __forceinline__ uint32_t level3_maps(const uint32_t (&w)[kFnvLaneBytes / 4], uint32_t low, uint32_t par) {
-    uint32_t r = low;
+    } else {
+        // two machines a register, half A's in byte 0 and half B's in byte 2, register m from m in the level's lowest bits
 #pragma unroll
-    for (int k = 0; k < kHalfWords; ++k)
+        for (uint32_t m = 0; m < kMachines; ++m) a[m] = low | ((m << kJ) * 0x00010001u);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) r = step_pair(r, pair_byte(w[k], w[kHalfWords + k], i));
-    return map2_of<6>(r & 0xFFu, par, 0u) | (map2_of<6>((r >> 16) & 0xFFu, par >> 16, 0u) << 16);
+        for (int k = 0; k < kHalfWords; ++k)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t word = i < 2 ? w[k] : w[kHalfWords + k], bb = (i & 1) ? word >> 8 : word;
+#pragma unroll
+                for (uint32_t& m : a) m = step_pair(m, bb);
+            }
+#pragma unroll
+        for (int m = 0; m < kMachines; ++m) b[m] = a[m] >> 16;
+    }
+    return map_of<kJ, kBits>(a, par, 0u) | (map_of<kJ, kBits>(b, par >> 16, 0u) << 16);
 }
 
 // ---- the gather fused with the hash -------------------------------------------------------------------------------
@@ -671,11 +754,11 @@ __device__ __forceinline__ bool gather_in_extent(const HashExtent& X, uint8_t* b
 // run or two issues its 16 loads at once from one or two bases; a segment over three runs or more, and the payload's
 // last partial segment, goes chunk by chunk into the payload, which the lane then reads back (its own stores, after a
 // fence).  The payload is written by store_wave below (the last partial segment only here).
-__device__ __forceinline__ void gather_segment(const HashMapArgs& m, uint8_t* base, uint32_t e_group, uint64_t begin,
+__device__ __forceinline__ void gather_segment(const HashExtent* ext, bool store, uint8_t* base, uint32_t e_group, uint64_t begin,
                                                uint64_t len, uint32_t (&w)[kFnvLaneBytes / 4]) {
     uint32_t e = e_group;
-    while (m.ext[e].end <= begin) ++e;
-    HashExtent x = m.ext[e];
+    while (ext[e].end <= begin) ++e;
+    HashExtent x = ext[e];
     uint8_t* dst = base + begin;   // `base` + o addresses payload byte o of this workgroup's segment
     const uint64_t seg_end = begin + len;
     const Run a = run_at(x, begin, dst);
@@ -685,7 +768,7 @@ __device__ __forceinline__ void gather_segment(const HashMapArgs& m, uint8_t* ba
         bool two = a.end >= seg_end;
         if (!two) {
             ka = uint32_t((a.end - begin) >> 4);
-            if (a.end >= x.end) x = m.ext[++e];
+            if (a.end >= x.end) x = ext[++e];
             b = run_at(x, a.end, dst + 16u * ka);
             two = b.end >= seg_end;
         }
@@ -696,16 +779,16 @@ __device__ __forceinline__ void gather_segment(const HashMapArgs& m, uint8_t* ba
         // three runs or more: walk from the workgroup's first extent again (the look-ahead above may have moved past
         // the extent holding `begin`)
         e = e_group;
-        while (m.ext[e].end <= begin) ++e;
-        x = m.ext[e];
+        while (ext[e].end <= begin) ++e;
+        x = ext[e];
     }
 #pragma unroll 1
     for (uint64_t o = begin; o < seg_end;) {
-        while (x.end <= o) x = m.ext[++e];
+        while (x.end <= o) x = ext[++e];
         const Run r = run_at(x, o, base + o);
         const uint64_t o0 = o, end = r.end < seg_end ? r.end : seg_end;
         for (; o < end; o += 16)
-            if (r.store && m.store) put16(base + o, r.src ? *(const gu32x4*) (r.src + (o - o0)) : u32x4{0u, 0u, 0u, 0u});
+            if (r.store && store) put16(base + o, r.src ? *(const gu32x4*) (r.src + (o - o0)) : u32x4{0u, 0u, 0u, 0u});
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");   // the lane's stores complete before its reads
     if (len == kFnvLaneBytes) load_segment(dst, w);
@@ -719,12 +802,12 @@ __device__ __forceinline__ void gather_segment(const HashMapArgs& m, uint8_t* ba
 // contiguous per instruction, non-temporal.  Bytes at or past `limit` (the part hashed in the kernel) are not written
 // here.
 constexpr int kXposeRow = kFnvLaneBytes / 16 + 1;   // chunks per LDS row: a lane's 16 and one of padding
-__device__ __forceinline__ void store_wave(u32x4 (&lds)[16 * kXposeRow], const uint32_t (&w)[kFnvLaneBytes / 4],
+__device__ __forceinline__ void store_wave(u32x4 (&lds)[8 * kXposeRow], const uint32_t (&w)[kFnvLaneBytes / 4],
                                            uint8_t* dst, uint64_t wave_begin, uint64_t limit, int lane) {
 #pragma unroll
-    for (int pass = 0; pass < 4; ++pass) {
-        if ((lane >> 4) == pass) {
-            const int row = (lane & 15) * kXposeRow;
+    for (int pass = 0; pass < 8; ++pass) {
+        if ((lane >> 3) == pass) {
+            const int row = (lane & 7) * kXposeRow;
 #pragma unroll
             for (int k = 0; k < kFnvLaneBytes / 16; ++k)
                 lds[row + k] = u32x4{w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]};
@@ -732,13 +815,17 @@ __device__ __forceinline__ void store_wave(u32x4 (&lds)[16 * kXposeRow], const u
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int c = r * 64 + lane;   // chunk of this pass's 4 KiB: lane c / 16's chunk c % 16
-            const u32x4 v = lds[(c >> 4) * kXposeRow + (c & 15)];
-            const uint64_t o = wave_begin + uint64_t(pass) * 4096u + uint64_t(c) * 16u;
-            // non-temporal: the fused 128K capture 2.75 against 2.79-2.81 ms with regular stores
-            if (o < limit) __builtin_nontemporal_store(v, (gu32x4*) (dst + o));
+        // step words 4c .. 4c + 3 of this pass's segment lane / 8 and their partners: chunk c of each half
+        const int seg = lane >> 3, c = lane & 7;
+        const u32x4 lo = lds[seg * kXposeRow + c], hi = lds[seg * kXposeRow + kHalfWords / 4 + c];
+        const u32x4 a = {low_halves(lo.x, hi.x), low_halves(lo.y, hi.y), low_halves(lo.z, hi.z), low_halves(lo.w, hi.w)};
+        const u32x4 b = {high_halves(lo.x, hi.x), high_halves(lo.y, hi.y), high_halves(lo.z, hi.z),
+                         high_halves(lo.w, hi.w)};
+        const uint64_t o = wave_begin + uint64_t(pass) * 2048u + uint64_t(seg) * kFnvLaneBytes + uint64_t(c) * 16u;
+        // non-temporal: the fused 128K capture 2.75 against 2.79-2.81 ms with regular stores
+        if (o < limit) {   // whole segments: both chunks
+            __builtin_nontemporal_store(a, (gu32x4*) (dst + o));
+            __builtin_nontemporal_store(b, (gu32x4*) (dst + o + kPairBytes));
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -746,146 +833,181 @@ __device__ __forceinline__ void store_wave(u32x4 (&lds)[16 * kXposeRow], const u
     }
 }
 
-// status: three arrays of `stride` words (one per level); ctl: [0] the ticket counter, [1] the fault word, [2..3] the
-// sum of the workgroups' sums (each workgroup adds its own with one 64-bit atomic).  kMapped: the payload is gathered
-// through `map` (stored, and hashed up to `n`, its whole lane segments) instead of read from `data`.  Not kMapped,
-// with `map.seg` set: the payload is read where its segments hold it (`data` unused).
-// Five waves per SIMD (the mapped instance would take 110 VGPRs and four; held to 96 it spills 5 words and runs the
-// fused 128K capture in 2.78-2.85 ms against 2.82 at four waves).  Every value the gather keeps live past its look-ahead
-// costs spills here: an extra extent index held across it spilled 35 words and took the capture to 3.03 ms.
-template <bool kMapped>
-__global__ void __launch_bounds__(kFnvThreads) __attribute__((amdgpu_waves_per_eu(5, 8))) fnv_onepass_kernel(const uint8_t* data, uint64_t n, bool aligned,
-                                                                uint64_t seed, const uint64_t* seed_dev,
-                                                                uint32_t* status, uint64_t stride, uint32_t* ctl,
-                                                                uint32_t spin_limit, HashMapArgs map,
-                                                                FnvCarries carries, uint64_t carry_count) {
+// kMapped: the payload is gathered through `map` (stored, and hashed up to `n`, its whole lane segments) instead of read
+// from `data`.  Not kMapped, with `map.seg` set: the payload is read where its segments hold it (`data` unused).
+// What bounds it: the two look-backs of a workgroup's 35 us, 6-7 us each of waiting for the latest of the workgroups before
+// it (about 2 us), the word's way through memory and the read's (about 3.5 us), and, at 70% busy vector units, its 17
+// operations per two bytes.  3.3 GB in 1.36 ms (1.76 ms with three levels and the sums on the vector units), checked
+// with carries in 0.87 (1.29), the 128K slot gathered and hashed in 1.76 (2.03).
+// Five waves per SIMD (96 VGPRs).  Taking several 64 KiB per workgroup, as the carried check does, measured slower here (3.3
+// GB in 1.60 ms): the workgroups' starts then spread over 3-5 us instead of 2, and every look-back waits for the latest.
+template <bool kMapped, bool kCarried>
+__global__ void __launch_bounds__(kFnvThreads) __attribute__((amdgpu_waves_per_eu(5, 8))) fnv_onepass_kernel(OnepassArgs) {
     __shared__ LevelLds L;
-    __shared__ uint32_t s_ticket;
-    __shared__ uint64_t s_sum[kFnvThreads / 64];
-    __shared__ u32x4 s_xpose[kMapped ? kFnvThreads / 64 : 1][16 * kXposeRow];
-    if (threadIdx.x == 0) s_ticket = atomicAdd(ctl, 1u);
-    __syncthreads();
-    const uint64_t g = uint32_t(__builtin_amdgcn_readfirstlane(int(s_ticket)));
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint64_t begin = (g * kFnvThreads + threadIdx.x) * kFnvLaneBytes;
-    const bool live = begin < n;
-    const uint64_t len = !live ? 0 : n - begin < kFnvLaneBytes ? n - begin : kFnvLaneBytes;
-    // the mapped instance hashes whole lane segments only (its launch passes n rounded down to them, the closing kernel
-    // takes the rest), so every live lane is whole there and the byte-at-a-time forms below drop out of it
-    const bool full = kMapped ? live : aligned && len == kFnvLaneBytes;
-    const uint8_t* p = data + begin;
-    if (!kMapped && map.seg) {
-        // a payload read where its segments hold it: this workgroup's 64 KiB lie in segment k
-        const uint64_t k = g * uint64_t(kFnvGroupBytes) / map.seg_bytes;
-        p = map.seg[k] + (begin - k * map.seg_bytes);
-    }
-    uint32_t* fault = ctl + 1;
-    uint32_t w[kFnvLaneBytes / 4] = {};
-    uint8_t* base = nullptr;   // mapped: `base` + o addresses payload byte o in the segment holding this workgroup's bytes
-    if constexpr (kMapped) {
-        // the workgroup's part of the map in one round trip: its 14 words read together through the constant address
-        // space (scalar loads; the map does not change during the launch) and held from here, rather than each field
-        // loaded in the branch that first needs it, one round trip after another
-        typedef const __attribute__((address_space(4))) uint64_t ConstWord;
-        const ConstWord* q = (const ConstWord*) (map.grp + g);
-        uint64_t h[14];
+    __shared__ u32x4 s_xpose[kMapped ? kFnvThreads / 64 : 1][8 * kXposeRow];
+    __shared__ u32x4 s_weights[kWeightChunks];
+    if (!kCarried && threadIdx.x == 0) L.ticket = atomicAdd(kernel_args()->ctl, 1u);
+    {
+        u32x4 weights[kWeightChunks / kFnvThreads];
 #pragma unroll
-        for (int i = 0; i < 14; ++i) h[i] = q[i];
-        asm volatile("" ::"s"(h[0]), "s"(h[1]), "s"(h[2]), "s"(h[3]), "s"(h[4]), "s"(h[5]), "s"(h[6]), "s"(h[7]),
-                     "s"(h[8]), "s"(h[9]), "s"(h[10]), "s"(h[11]), "s"(h[12]), "s"(h[13]));
-        HashGroup hg;
-        static_assert(offsetof(HashGroup, pad) == 14 * 8, "the words read are the group's fields");
-        __builtin_memcpy(&hg, h, sizeof(h));
-        base = hg.base;
-        if (begin < map.n_total) {
-            const uint64_t wave_lo = (g * kFnvThreads + uint64_t(wave) * 64) * kFnvLaneBytes;
-            const uint64_t wave_hi = wave_lo + 64u * kFnvLaneBytes;
-            bool done = false;
-            if (hg.two && wave_hi <= map.n_total) {   // every lane of the wave whole, inside one of the two extents
-                if (wave_hi <= hg.x[0].end)
-                    done = gather_in_extent(hg.x[0], base, begin, w);
-                else if (wave_lo >= hg.x[0].end)
-                    done = gather_in_extent(hg.x[1], base, begin, w);
-            }
-            if (!done) {
-                const uint64_t left = map.n_total - begin;
-                gather_segment(map, base, hg.first, begin, left < kFnvLaneBytes ? left : kFnvLaneBytes, w);
-            }
+        for (int i = 0; i < kWeightChunks / kFnvThreads; ++i)
+            weights[i] = ((const gu32x4*) &g_sum_weights.w[0][0][0])[i * kFnvThreads + threadIdx.x];
+#pragma unroll
+        for (int i = 0; i < kWeightChunks / kFnvThreads; ++i) s_weights[i * kFnvThreads + threadIdx.x] = weights[i];
+    }
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    __syncthreads();
+    uint64_t total = 0, total_part = 0;   // thread 0: the workgroup's sums
+    uint32_t g = kCarried ? blockIdx.x : __builtin_amdgcn_readfirstlane(L.ticket);
+#pragma unroll 1
+    do {
+        const int lane = lane_id();
+        // the lane's segment: its first byte, and whether it is whole (and aligned), partial or past the input.  The
+        // mapped instance hashes whole lane segments only (its launch passes n rounded down to them, the closing kernel
+        // takes the rest), so the byte-at-a-time forms drop out of it
+        const auto begin_of = [&] { return ((uint64_t(g) * kFnvThreads + uint32_t(wave) * 64u) + uint32_t(lane)) * kFnvLaneBytes; };
+        const auto bytes_of = [&] {
+            const uint64_t begin = begin_of(), n = kernel_args()->n;
+            return begin >= n ? 0u : n - begin < kFnvLaneBytes ? uint32_t(n - begin) : uint32_t(kFnvLaneBytes);
+        };
+        const auto address_of = [&]() -> const uint8_t* {
+            ConstArgs* a = kernel_args();
+            const uint64_t begin = begin_of();
+            if (!a->map.seg) return a->data + begin;
+            // a payload read where its segments hold it: this workgroup's 64 KiB lie in segment k
+            const uint64_t k = uint64_t(g) * kFnvGroupBytes / a->map.seg_bytes;
+            return a->map.seg[k] + (begin - k * a->map.seg_bytes);
+        };
+        const uint32_t len = bytes_of();
+        const bool full = kMapped ? len != 0u : len == kFnvLaneBytes && kernel_args()->aligned;
+        const bool bytes = !kMapped && !full && len != 0u;
+        // a check's carries around this workgroup
+        uint32_t before = 0, after = 0;
+        if constexpr (kCarried) {
+            ConstArgs* a = kernel_args();
+            before = g > 0 ? uint32_t(a->carries.in[g - 1]) : start_byte();
+            after = g < a->carry_count ? uint32_t(a->carries.in[g]) : 0x100u;
         }
-    } else if (full) {
-        load_segment(p, w);
-    }
-    const uint64_t h0 = start_state(seed, seed_dev);
-
-    // the three levels: every lane's map of the level (a whole segment from its two halves in registers, a partial or
-    // unaligned one a byte at a time), then the workgroup's look-back.  `s` gathers the true start bits at the lane's
-    // segment, `sb` at its midpoint (its first half's map applied to the level's start bits)
-    const uint32_t par = full ? half_parities(w) : 0u;
-    uint32_t halves = 0, lane_map = 0;
-    if (full) {
-        halves = level1_maps(w, par);
-        lane_map = compose<3>(halves >> 16, halves & 0xFFFFu);
-    } else if (live) {
-        lane_map = map3_bytes<0>(p, len, 0u);
-    }
-    // the gathered payload is written while the last look-back waits: 2.05 ms for the 128K capture + hash, against
-    // 2.22 ms while the first waits, 2.15 ms while the second waits and 2.18 ms after the last (stores issued earlier
-    // meet the next workgroups' gathers)
-    const auto store_gathered = [&] {
-        if constexpr (kMapped)
-            if (map.store)
-                store_wave(s_xpose[wave], w, base, (g * kFnvThreads + uint64_t(wave) * 64) * kFnvLaneBytes, n, lane);
-    };
-    uint32_t end_bits = 0;   // wave 0: the workgroup's end state, level by level (its carry)
-    uint32_t s = resolve_level<3>(wave, lane_map, g, status, uint32_t(h0) & 7u, fault, spin_limit, L,
-                                  kFirstSleeps, [] {}, 0, carries.in, carry_count, end_bits);
-    uint32_t sb = apply<3>(halves & 0xFFFFu, s);
-
-    lane_map = 0;
-    if (full) {
-        halves = level2_maps(w, s | (sb << 16), par);
-        lane_map = compose<3>(halves >> 16, halves & 0xFFFFu);
-    } else if (live) {
-        lane_map = map3_bytes<3>(p, len, s);
-    }
-    uint32_t st = resolve_level<3>(wave, lane_map, g, status + stride, uint32_t(h0 >> 3) & 7u, fault, spin_limit, L,
-                                   kFirstSleeps, [] {}, 3, carries.in, carry_count, end_bits);
-    s |= st << 3;
-    sb |= apply<3>(halves & 0xFFFFu, st) << 3;
-
-    lane_map = 0;
-    if (full) {
-        halves = level3_maps(w, s | (sb << 16), par);
-        lane_map = compose<2>(halves >> 16, halves & 0xFFFFu);
-    } else if (live) {
-        lane_map = map2_bytes<6>(p, len, s);
-    }
-    st = resolve_level<2>(wave, lane_map, g, status + 2 * stride, uint32_t(h0 >> 6) & 3u, fault, spin_limit, L,
-                          kMapped ? kFirstSleepsMapped : kFirstSleeps, store_gathered, 6, carries.in, carry_count,
-                          end_bits);
-    if (carries.out && threadIdx.x == 0 && g < carry_count) carries.out[g] = uint8_t(end_bits);
-    s |= st << 6;
-    sb |= apply<2>(halves & 0xFFFFu, st) << 6;
-
-    // the Horner sums, from the true low bytes at the segment's start and midpoint
-    uint64_t acc = 0;
-    if (full) {
-        // p^(n - r), r the end of the wave's last segment: wave-uniform.  p has order dividing 2^62 modulo 2^64, so
-        // the exponent is taken modulo 2^62 (r passes n in the buffer's last wave)
-        const uint64_t wave_end = ((g * kFnvThreads) + uint64_t(wave) * 64 + 64) * kFnvLaneBytes;
-        const uint64_t wave_pow = pow_prime((n - wave_end) & ((uint64_t(1) << 62) - 1));
-        acc = halves_sum(w, s | (sb << 16)) * kLanePow.v[lane] * wave_pow;
-    } else if (live) {
-        acc = segment_sum(p, n, begin, s);
-    }
-    for (int m = 32; m > 0; m >>= 1) acc += shfl_xor64(acc, m);
-    if (lane == 0) s_sum[wave] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint64_t sum = 0;
+        // what the workgroup's sum is worth where the last one ends; read here, with the data, rather than when the sum is
+        // there and everything else done
+        const uint32_t rest = kernel_args()->groups - 1u - g;
+        const uint64_t worth = group_pow(0, rest) * group_pow(1, rest) * group_pow(2, rest) * group_pow(3, rest);
+        uint32_t w[kFnvLaneBytes / 4] = {};
+        uint8_t* base = nullptr;   // mapped: `base` + o addresses payload byte o in the segment holding this workgroup's bytes
+        if constexpr (kMapped) {
+            // the workgroup's part of the map in one round trip: its 14 words read together through the constant address
+            // space (scalar loads; the map does not change during the launch) and held from here, rather than each field
+            // loaded in the branch that first needs it, one round trip after another
+            typedef const __attribute__((address_space(4))) uint64_t ConstWord;
+            ConstArgs* a = kernel_args();
+            const ConstWord* q = (const ConstWord*) (a->map.grp + g);
+            uint64_t h[14];
 #pragma unroll
-        for (int k = 0; k < kFnvThreads / 64; ++k) sum += s_sum[k];
-        atomicAdd(reinterpret_cast<unsigned long long*>(ctl + 2), (unsigned long long) sum);
+            for (int i = 0; i < 14; ++i) h[i] = q[i];
+            asm volatile("" ::"s"(h[0]), "s"(h[1]), "s"(h[2]), "s"(h[3]), "s"(h[4]), "s"(h[5]), "s"(h[6]), "s"(h[7]),
+                         "s"(h[8]), "s"(h[9]), "s"(h[10]), "s"(h[11]), "s"(h[12]), "s"(h[13]));
+            HashGroup hg;
+            static_assert(offsetof(HashGroup, pad) == 14 * 8, "the words read are the group's fields");
+            __builtin_memcpy(&hg, h, sizeof(h));
+            base = hg.base;
+            const uint64_t begin = begin_of(), n_total = a->map.n_total;
+            if (begin < n_total) {
+                const uint64_t wave_lo = (uint64_t(g) * kFnvThreads + uint64_t(wave) * 64) * kFnvLaneBytes;
+                const uint64_t wave_hi = wave_lo + 64u * kFnvLaneBytes;
+                bool done = false;
+                if (hg.two && wave_hi <= n_total) {   // every lane of the wave whole, inside one of the two extents
+                    if (wave_hi <= hg.x[0].end)
+                        done = gather_in_extent(hg.x[0], base, begin, w);
+                    else if (wave_lo >= hg.x[0].end)
+                        done = gather_in_extent(hg.x[1], base, begin, w);
+                }
+                if (!done) {
+                    const uint64_t left = n_total - begin;
+                    gather_segment(a->map.ext, a->map.store, base, hg.first, begin,
+                                   left < kFnvLaneBytes ? left : kFnvLaneBytes, w);
+                }
+            }
+        } else if (full) {
+            load_segment(address_of(), w);
+        }
+        pair_words(w);
+
+        // the levels: every lane's map of the level (a whole segment from its two halves in registers, a partial or unaligned
+        // one a byte at a time), then the workgroup's start state.  `s` gathers the true start bits at the lane's segment,
+        // `sb` at its midpoint (its first half's map applied to the level's start bits)
+        const uint32_t par = full ? half_parities(w) : 0u;
+        uint32_t s = 0, sb = 0, end_bits = 0;   // end_bits: the workgroup's end state, level by level (its carry)
+        const auto level = [&](auto index, auto first_bit, auto width, int first_sleeps, auto during) {
+            constexpr int kLevel = decltype(index)::value, kJ = decltype(first_bit)::value, kBits = decltype(width)::value;
+            uint32_t halves = 0, lane_map = 0;
+            if constexpr (kLevel > 0) renew_words(w);
+            if (full) {
+                halves = level_maps<kJ, kBits>(w, s | (sb << 16), par);
+                lane_map = compose<kBits>(halves >> 16, halves & map_mask<kBits>());
+            } else if (bytes) {
+                lane_map = map_bytes<kJ, kBits>(address_of(), bytes_of(), s);
+            }
+            const uint32_t st = resolve_level<kCarried, kLevel, kJ, kBits>(wave, lane_map, g, L, first_sleeps, during, before,
+                                                                           end_bits);
+            s |= st << kJ;
+            sb |= apply<kBits>(halves & map_mask<kBits>(), st) << kJ;
+        };
+        if constexpr (kCarried) {
+            level(Int<0>{}, Int<0>{}, Int<3>{}, 0, [] {});
+            level(Int<1>{}, Int<3>{}, Int<3>{}, 0, [] {});
+            level(Int<2>{}, Int<6>{}, Int<2>{}, 0, [] {});
+        } else {
+            level(Int<0>{}, Int<0>{}, Int<4>{}, kFirstSleeps, [] {});
+            // the gathered payload is written while the last look-back waits (stores issued earlier meet the next
+            // workgroups' gathers, later ones hold up the workgroup's end)
+            level(Int<1>{}, Int<4>{}, Int<4>{}, kMapped ? kFirstSleepsMapped : kFirstSleeps, [&] {
+                if constexpr (kMapped) {
+                    ConstArgs* a = kernel_args();
+                    if (a->map.store)
+                        store_wave(s_xpose[wave], w, base, (uint64_t(g) * kFnvThreads + uint64_t(wave) * 64) * kFnvLaneBytes,
+                                   a->n, lane);
+                }
+            });
+        }
+        if (wave == 0 && lane == 0) {
+            ConstArgs* a = kernel_args();
+            if (a->carries.out && g < a->carry_count) a->carries.out[g] = uint8_t(end_bits);
+            if (kCarried && after != 0x100u && end_bits != after) flag_fault(a->ctl + 1, kFaultCarry);
+        }
+
+        // the sums, from the true low bytes at the segment's start and midpoint: the wave's whole segments together
+        // (relative to the end of its last segment), a partial or unaligned one a byte at a time
+        renew_words(w);
+        uint64_t acc = 0;
+        if (__ballot(full)) acc = wave_sum(w, full ? s | (sb << 16) : 0u, lane, s_weights);
+        for (int m = 32; m > 0; m >>= 1) acc += shfl_xor64(acc, m);
+        uint64_t part = 0;
+        if (!kMapped && __ballot(bytes)) {
+            if (bytes) part = segment_sum(address_of(), kernel_args()->n, begin_of(), s);
+            for (int m = 32; m > 0; m >>= 1) part += shfl_xor64(part, m);
+        }
+        if (lane == 0) {
+            L.sum[wave] = acc;
+            L.part[wave] = part;
+        }
+        __syncthreads();
+        if (wave == 0 && lane == 0) {
+            constexpr uint64_t wave_pow = prime_pow_of(64u * kFnvLaneBytes);
+            uint64_t sum = 0, parts = 0;
+#pragma unroll
+            for (int q = 0; q < kFnvThreads / 64; ++q) {
+                sum = sum * wave_pow + L.sum[q];
+                parts += L.part[q];
+            }
+            total += sum * worth;
+            total_part += parts;
+        }
+        g += gridDim.x;
+    } while (kCarried && g < kernel_args()->groups);
+    if (threadIdx.x == 0) {
+        uint32_t* ctl = kernel_args()->ctl;
+        atomicAdd(reinterpret_cast<unsigned long long*>(ctl + 2), (unsigned long long) total);
+        if (total_part) atomicAdd(reinterpret_cast<unsigned long long*>(ctl + 4), (unsigned long long) total_part);
     }
 }
 
@@ -894,14 +1016,14 @@ __global__ void __launch_bounds__(kFnvThreads) __attribute__((amdgpu_waves_per_e
 __global__ void __launch_bounds__(kThreads) fnv_onepass_init_kernel(uint32_t* status, uint64_t words, uint32_t* ctl) {
     const uint64_t stride = uint64_t(gridDim.x) * kThreads;
     for (uint64_t i = uint64_t(blockIdx.x) * kThreads + threadIdx.x; i < words; i += stride) status[i] = 0u;
-    if (blockIdx.x == 0 && threadIdx.x < 4) ctl[threadIdx.x] = 0u;
+    if (blockIdx.x == 0 && threadIdx.x < 6) ctl[threadIdx.x] = 0u;
 }
 }  // namespace
 
 // The bound on each look-back wait, in window reads; tests lower it to force a wait to run out.
 std::atomic<uint32_t> g_spin_limit{kSpinLimit};
 
-// Workspace: [ticket, fault and sum words][status words: three levels of `stride` words].
+// Workspace: [ticket, fault and sum words][status words: up to three per workgroup].
 FnvWorkspace fnv_workspace(uint64_t n) {
     FnvWorkspace w{};
     w.segments = (n + kFnvLaneBytes - 1) / kFnvLaneBytes;
@@ -909,34 +1031,49 @@ FnvWorkspace fnv_workspace(uint64_t n) {
     auto up = [](uint64_t x) { return (x + 255) / 256 * 256; };
     w.off_ctl = 0;
     w.off_status = 256;
-    w.stride = up(w.groups * 4) / 4;
-    w.bytes = w.off_status + 3 * w.stride * 4;
+    w.bytes = w.off_status + 3 * up(w.groups * 4);
     return w;
+}
+
+// Clears a launch's words and enqueues the one-pass kernel over `a` (its ctl, status, groups, turns and spin limit set
+// here); returns ctl, or null for an empty input, which needs neither.
+template <bool kMapped>
+uint32_t* enqueue_onepass(OnepassArgs a, uint8_t* workspace, uint64_t bytes, hipStream_t stream) {
+    const FnvWorkspace w = fnv_workspace(bytes);
+    if (!w.groups) return nullptr;
+    a.ctl = reinterpret_cast<uint32_t*>(workspace + w.off_ctl);
+    a.status = reinterpret_cast<uint32_t*>(workspace + w.off_status);
+    a.groups = uint32_t(w.groups);
+    a.spin_limit = g_spin_limit.load();
+    const uint64_t words = kStatusWords * w.groups, init_blocks = (words + kThreads - 1) / kThreads < 1024 ? (words + kThreads - 1) / kThreads : 1024;
+    hipLaunchKernelGGL(fnv_onepass_init_kernel, dim3(unsigned(init_blocks)), dim3(kThreads), 0, stream, a.status, words, a.ctl);
+    if (!kMapped && a.carries.in) {
+        // no workgroup waits for another: each takes up to four 64 KiB in turn, which spares it the start of a workgroup
+        // (3.3 GB checked in 0.88 ms against 1.35 ms with one each, and alike with eight) while others' kernels still get
+        // their turn on the CUs; fewer when that would leave some of the 1280 (five per CU) without work
+        const uint32_t turns = a.groups < 2 * 1280 ? 1 : a.groups < 4 * 1280 ? a.groups / 1280 : 4;
+        hipLaunchKernelGGL((fnv_onepass_kernel<false, true>), dim3((a.groups + turns - 1) / turns), dim3(kFnvThreads), 0, stream, a);
+    } else {
+        hipLaunchKernelGGL((fnv_onepass_kernel<kMapped, false>), dim3(a.groups), dim3(kFnvThreads), 0, stream, a);
+    }
+    return a.ctl;
 }
 
 hipError_t launch_fnv1a64(const void* data, uint64_t n, uint64_t seed, const uint64_t* seed_dev, uint64_t* out,
                           uint32_t* fault_out, void* workspace, hipStream_t stream, uint64_t expected, uint32_t* verdict,
                           const FnvCarries& carries) {
-    const FnvWorkspace w = fnv_workspace(n);
-    uint8_t* ws = static_cast<uint8_t*>(workspace);
-    const uint8_t* src = static_cast<const uint8_t*>(data);
-    const bool aligned = (reinterpret_cast<uintptr_t>(data) & 15u) == 0;
-    uint32_t* ctl = reinterpret_cast<uint32_t*>(ws + w.off_ctl);
-    uint32_t* status = reinterpret_cast<uint32_t*>(ws + w.off_status);
-    if (w.groups > 0) {
-        const uint64_t words = 3 * w.stride;
-        const uint64_t init_blocks = (words + kThreads - 1) / kThreads < 1024 ? (words + kThreads - 1) / kThreads : 1024;
-        hipLaunchKernelGGL(fnv_onepass_init_kernel, dim3(unsigned(init_blocks)), dim3(kThreads), 0, stream, status, words,
-                           ctl);
-        hipLaunchKernelGGL(fnv_onepass_kernel<false>, dim3(unsigned(w.groups)), dim3(kFnvThreads), 0, stream, src, n, aligned,
-                           seed, seed_dev, status, w.stride, ctl, g_spin_limit.load(), HashMapArgs{}, carries,
-                           fnv_carry_count(n));
-    }
+    OnepassArgs a{};
+    a.data = static_cast<const uint8_t*>(data);
+    a.n = n;
+    a.aligned = (reinterpret_cast<uintptr_t>(data) & 15u) == 0;
+    a.seed = seed;
+    a.seed_dev = seed_dev;
+    a.carries = carries;
+    a.carry_count = fnv_carry_count(n);
+    const uint32_t* ctl = enqueue_onepass<false>(a, static_cast<uint8_t*>(workspace), n, stream);
     // the finish reads the start state before it writes `out`, so `out` may be `seed_dev` itself
-    const bool any = w.groups > 0;
-    hipLaunchKernelGGL(fnv_finish_kernel, dim3(1), dim3(1), 0, stream, any ? reinterpret_cast<const uint64_t*>(ctl + 2) : nullptr,
-                       seed, seed_dev, n, out, fault_out, seed_dev != nullptr, expected, verdict, any ? ctl + 1 : nullptr,
-                       nullptr, 0u);
+    hipLaunchKernelGGL(fnv_finish_kernel, dim3(1), dim3(1), 0, stream, ctl, seed, seed_dev, n, out, fault_out,
+                       seed_dev != nullptr, expected, verdict, nullptr, 0u);
     return hipGetLastError();
 }
 
@@ -984,41 +1121,19 @@ hipError_t launch_fnv1a64_mapped(const HashMapArgs& map, const uint8_t* tail, ui
                                  uint32_t* verdict, const FnvCarries& carries) {
     const uint64_t n_total = map.n_total, n_full = n_total & ~uint64_t(kFnvLaneBytes - 1);
     if (n_total % 16) return hipErrorInvalidValue;   // maps hold whole 16-byte chunks (the closing kernel loads them)
-    const FnvWorkspace w = fnv_workspace(n_total);
+    OnepassArgs a{};
+    a.aligned = 1u;
+    a.seed = seed;
+    a.map = map;
+    a.carries = carries;
+    a.carry_count = fnv_carry_count(n_total);
     uint8_t* ws = static_cast<uint8_t*>(workspace);
-    uint32_t* ctl = reinterpret_cast<uint32_t*>(ws + w.off_ctl);
-    uint32_t* status = reinterpret_cast<uint32_t*>(ws + w.off_status);
-    if (!map.store) {
-        // a map that only reads: the plain kernel hashes the payload where its segments hold it, the last partial
-        // lane segment included (no gather, so nothing waits for bytes to be placed)
-        if (w.groups > 0) {
-            const uint64_t words = 3 * w.stride;
-            const uint64_t init_blocks = (words + kThreads - 1) / kThreads < 1024 ? (words + kThreads - 1) / kThreads : 1024;
-            hipLaunchKernelGGL(fnv_onepass_init_kernel, dim3(unsigned(init_blocks)), dim3(kThreads), 0, stream, status,
-                               words, ctl);
-            hipLaunchKernelGGL(fnv_onepass_kernel<false>, dim3(unsigned(w.groups)), dim3(kFnvThreads), 0, stream, nullptr,
-                               n_total, true, seed, nullptr, status, w.stride, ctl, g_spin_limit.load(), map, carries,
-                               fnv_carry_count(n_total));
-        }
-        const bool any = w.groups > 0;
-        hipLaunchKernelGGL(fnv_finish_kernel, dim3(1), dim3(1), 0, stream,
-                           any ? reinterpret_cast<const uint64_t*>(ctl + 2) : nullptr, seed, nullptr, n_total, out,
-                           fault_out, false, expected, verdict, any ? ctl + 1 : nullptr, nullptr, 0u);
-        return hipGetLastError();
-    }
-    if (w.groups > 0) {
-        const uint64_t words = 3 * w.stride;
-        const uint64_t init_blocks = (words + kThreads - 1) / kThreads < 1024 ? (words + kThreads - 1) / kThreads : 1024;
-        hipLaunchKernelGGL(fnv_onepass_init_kernel, dim3(unsigned(init_blocks)), dim3(kThreads), 0, stream, status, words,
-                           ctl);
-        hipLaunchKernelGGL(fnv_onepass_kernel<true>, dim3(unsigned(w.groups)), dim3(kFnvThreads), 0, stream, nullptr, n_full,
-                           true, seed, nullptr, status, w.stride, ctl, g_spin_limit.load(), map, carries,
-                           fnv_carry_count(n_total));
-    }
-    const bool any = w.groups > 0;
-    hipLaunchKernelGGL(fnv_finish_kernel, dim3(1), dim3(1), 0, stream, any ? reinterpret_cast<const uint64_t*>(ctl + 2) : nullptr,
-                       seed, nullptr, n_full, out, fault_out, false, expected, verdict, any ? ctl + 1 : nullptr,
-                       tail, uint32_t(n_total - n_full));
+    // a map that only reads: the plain kernel hashes the payload where its segments hold it, the last partial lane segment
+    // included (no gather, so nothing waits for bytes to be placed)
+    a.n = map.store ? n_full : n_total;
+    const uint32_t* ctl = map.store ? enqueue_onepass<true>(a, ws, n_total, stream) : enqueue_onepass<false>(a, ws, n_total, stream);
+    hipLaunchKernelGGL(fnv_finish_kernel, dim3(1), dim3(1), 0, stream, ctl, seed, nullptr, a.n, out, fault_out, false, expected,
+                       verdict, map.store ? tail : nullptr, uint32_t(n_total - a.n));
     return hipGetLastError();
 }
 
