@@ -54,8 +54,6 @@ hipError_t launch_fnv1a64(const void* data, uint64_t n, uint64_t seed, const uin
 hipError_t launch_fnv1a64_mapped(const HashMapArgs& map, const uint8_t* tail, uint64_t seed, uint64_t* out,
                                  uint32_t* fault_out, void* workspace, hipStream_t stream, uint64_t expected = 0,
                                  uint32_t* verdict = nullptr, const FnvCarries& carries = {});
-hipError_t launch_hash_groups(const HashExtent* ext, uint32_t n_ext, uint64_t bytes, uint8_t* const* segs,
-                              uint32_t n_segs, uint64_t seg_bytes, HashGroup* grp, uint64_t groups, hipStream_t stream);
 
 static uint64_t host_mix64(uint64_t z) {
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -93,8 +91,8 @@ struct sc_plan {
 };
 
 struct sc_hash_map {
-    sc::HashExtent* ext_dev = nullptr;   // one device block: the extents, the workgroups' parts, the segments
-    sc::HashGroup* grp_dev = nullptr;
+    sc::HashExtent* ext_dev = nullptr;   // one device block: the extents, the segments
+    uint32_t n_ext = 0;
     uint8_t** seg_dev = nullptr;
     uint64_t seg_bytes = 0;
     const uint8_t* tail = nullptr;       // device address of the payload's last partial lane segment
@@ -1555,45 +1553,43 @@ int segment_list(const sc_segments* s, uint64_t bytes, std::vector<uint8_t*>& se
     return SC_OK;
 }
 
-// Makes a map in one device block: the extents and the segment table uploaded, each workgroup's part (sc::HashGroup)
-// built from them on the device (hash_groups_kernel), waited for before the map is handed out.  A map that only reads
-// (no extents) is hashed by the plain kernel from the segment table alone, so it needs nothing else.
+// Makes a map in one device block: the extents and the segment table uploaded (a launch finds each workgroup's extents
+// itself).  A map that only reads has no extents.
 int make_hash_map(const std::vector<sc::HashExtent>& ext, uint64_t bytes, const std::vector<uint8_t*>& segs,
                   uint64_t seg_bytes, bool store, sc_hash_map** out) {
-    const sc::FnvWorkspace w = sc::fnv_workspace(bytes);
-    const uint64_t n_grp = store ? std::max<uint64_t>(w.groups, 1) : 1;
     if (ext.size() >= (uint64_t(1) << 32) || segs.empty())
         return fail(SC_ERANGE, "sc_handoff: a hash map holds fewer than 2^32 extents and at least one segment");
     auto* m = new (std::nothrow) sc_hash_map();
     if (!m) return fail(SC_ENOMEM, "sc_handoff: hash map allocation failed");
     const uint64_t ext_bytes = round_up(ext.size() * sizeof(sc::HashExtent), 256);
-    const uint64_t grp_bytes = round_up(n_grp * sizeof(sc::HashGroup), 256);
-    hipError_t err = hipMalloc(reinterpret_cast<void**>(&m->ext_dev), ext_bytes + grp_bytes + segs.size() * 8);
+    hipError_t err = hipMalloc(reinterpret_cast<void**>(&m->ext_dev), ext_bytes + segs.size() * 8);
     if (err != hipSuccess) {
         delete m;
         return fail(SC_ENOMEM, std::string("sc_handoff: hash map: ") + hipGetErrorString(err));
     }
     uint8_t* block = reinterpret_cast<uint8_t*>(m->ext_dev);
-    m->grp_dev = reinterpret_cast<sc::HashGroup*>(block + ext_bytes);
-    m->seg_dev = reinterpret_cast<uint8_t**>(block + ext_bytes + grp_bytes);
+    m->seg_dev = reinterpret_cast<uint8_t**>(block + ext_bytes);
     if (!ext.empty()) err = hipMemcpy(m->ext_dev, ext.data(), ext.size() * sizeof(sc::HashExtent), hipMemcpyHostToDevice);
     if (err == hipSuccess) err = hipMemcpy(m->seg_dev, segs.data(), segs.size() * 8, hipMemcpyHostToDevice);
-    if (err == hipSuccess && store && !ext.empty())
-        err = sc::launch_hash_groups(m->ext_dev, uint32_t(ext.size()), bytes, m->seg_dev, uint32_t(segs.size()),
-                                     seg_bytes, m->grp_dev, w.groups, nullptr);
-    if (err == hipSuccess) err = hipStreamSynchronize(nullptr);
     if (err != hipSuccess) {
         (void) hipFree(m->ext_dev);
         delete m;
         return hip_fail(err, "hash map upload");
     }
     const uint64_t n_full = bytes & ~uint64_t(sc::kFnvLaneBytes - 1);
+    m->n_ext = uint32_t(ext.size());
     m->seg_bytes = seg_bytes;
     m->tail = segs[size_t(std::min<uint64_t>(n_full / seg_bytes, segs.size() - 1))] + n_full % seg_bytes;
     m->bytes = bytes;
     m->store = store;
     *out = m;
     return ok();
+}
+
+sc::HashMapArgs map_args(const sc_hash_map* map) {
+    const uint64_t pieces = map->seg_bytes / uint64_t(sc::kFnvGroupBytes);   // of a segment; one holds any payload from 2^31
+    return {map->ext_dev,   map->n_ext, map->store ? 1u : 0u, map->seg_dev, map->seg_bytes,
+            sc::make_fastdiv(uint32_t(std::min<uint64_t>(pieces, uint64_t(1) << 31))), map->bytes};
 }
 
 int hash_map_args(const sc_hash_map* map, const uint32_t* fault, const void* workspace, uint64_t workspace_bytes) {
@@ -1650,7 +1646,7 @@ int sc_hash_map_launch(const sc_hash_map* map, uint64_t seed, uint64_t* out, uin
                        uint64_t workspace_bytes, void* stream) {
     if (const int rc = hash_map_args(map, fault, workspace, workspace_bytes)) return rc;
     if (!out || !fault) return fail(SC_EINVAL, "sc_handoff: missing hash output or fault word");
-    const sc::HashMapArgs a{map->ext_dev, map->grp_dev, map->seg_dev, map->seg_bytes, map->bytes, map->store ? 1u : 0u};
+    const sc::HashMapArgs a = map_args(map);
     const hipError_t e =
         sc::launch_fnv1a64_mapped(a, map->tail, seed, out, fault, workspace, static_cast<hipStream_t>(stream));
     return e == hipSuccess ? ok() : hip_fail(e, "mapped hash launch");
@@ -1661,7 +1657,7 @@ int sc_hash_map_check_async(const sc_hash_map* map, uint64_t seed, uint64_t expe
     if (const int rc = hash_map_args(map, fault, workspace, workspace_bytes)) return rc;
     if (!out || !verdict || (reinterpret_cast<uintptr_t>(verdict) & 3u))
         return fail(SC_EINVAL, "sc_handoff: missing hash output, or a verdict word that is not 4-byte aligned");
-    const sc::HashMapArgs a{map->ext_dev, map->grp_dev, map->seg_dev, map->seg_bytes, map->bytes, map->store ? 1u : 0u};
+    const sc::HashMapArgs a = map_args(map);
     const hipError_t e = sc::launch_fnv1a64_mapped(a, map->tail, seed, out, fault, workspace,
                                                    static_cast<hipStream_t>(stream), expected, verdict);
     return e == hipSuccess ? ok() : hip_fail(e, "mapped hash launch");
@@ -1672,7 +1668,7 @@ int sc_hash_map_launch_carry(const sc_hash_map* map, uint64_t seed, uint64_t* ou
     if (const int rc = hash_map_args(map, fault, workspace, workspace_bytes)) return rc;
     if (!out || !fault) return fail(SC_EINVAL, "sc_handoff: missing hash output or fault word");
     if (!carry_out && sc::fnv_carry_count(map->bytes)) return fail(SC_EINVAL, "sc_handoff: missing carry output");
-    const sc::HashMapArgs a{map->ext_dev, map->grp_dev, map->seg_dev, map->seg_bytes, map->bytes, map->store ? 1u : 0u};
+    const sc::HashMapArgs a = map_args(map);
     sc::FnvCarries c;
     c.out = carry_out;
     const hipError_t e = sc::launch_fnv1a64_mapped(a, map->tail, seed, out, fault, workspace,
@@ -1689,7 +1685,7 @@ int sc_hash_map_check_carried_async(const sc_hash_map* map, uint64_t seed, uint6
     if (!carry && sc::fnv_carry_count(map->bytes)) return fail(SC_EINVAL, "sc_handoff: missing carries");
     if (map->store)
         return fail(SC_EINVAL, "sc_handoff: a check with carries reads the payload where it lies (sc_hash_map_create_read)");
-    const sc::HashMapArgs a{map->ext_dev, map->grp_dev, map->seg_dev, map->seg_bytes, map->bytes, 0u};
+    const sc::HashMapArgs a = map_args(map);
     sc::FnvCarries c;
     c.in = carry;
     const hipError_t e = sc::launch_fnv1a64_mapped(a, map->tail, seed, out, fault, workspace,

@@ -476,6 +476,13 @@ __device__ __forceinline__ ConstArgs* kernel_args() {
     asm volatile("" : "+s"(p));
     return p;
 }
+// Where the payload's segments put payload byte 0 of workgroup g's 64 KiB, which lie in one of them: `base` + o addresses
+// payload byte o.
+__device__ __forceinline__ uint8_t* payload_base(uint32_t g) {
+    ConstArgs* a = kernel_args();
+    const uint32_t k = uint32_t((uint64_t(__umulhi(g, a->map.seg_div.m)) + g) >> a->map.seg_div.s);
+    return a->map.seg[k] - uint64_t(k) * a->map.seg_bytes;
+}
 // The low byte the hash starts from.
 __device__ __forceinline__ uint32_t start_byte() {
     ConstArgs* a = kernel_args();
@@ -697,19 +704,26 @@ __device__ __forceinline__ Run run_at(const HashExtent& x, uint64_t o, uint8_t* 
     return r;
 }
 
-__device__ u32x4 g_hash_zero_chunk;   // read for zero runs, so every chunk takes the same load
+// Read for zero runs and by lanes past the payload's whole segments, so that every lane takes the same loads.
+__device__ u32x4 g_hash_zeros[kFnvLaneBytes / 16];
 
-// A lane's 256-byte segment from run a (its first ka chunks) and run b (the rest): 16 loads issued at once, a zero run's
-// from one zero chunk.
-__device__ __forceinline__ void load_runs(const Run& a, const Run& b, uint32_t ka, uint32_t (&w)[kFnvLaneBytes / 4]) {
-    const uint8_t* za = a.src ? a.src : reinterpret_cast<const uint8_t*>(&g_hash_zero_chunk);
-    const uint8_t* zb = b.src ? b.src : reinterpret_cast<const uint8_t*>(&g_hash_zero_chunk);
-    const uint64_t sa = a.src ? 16u : 0u, sb = b.src ? 16u : 0u;
+// Where a lane's segment is gathered from: chunk k at (k < ka ? a : b) + 16 k.  Every kind of extent comes down to one or
+// two contiguous runs, and the loads stand once, after them: with loads of their own in each branch the 64 registers they
+// meet in did not line up, and every path stored a chunk to scratch and read it back before the first level.
+struct SegmentSource {
+    const uint8_t* a;
+    const uint8_t* b;
+    uint32_t ka;
+};
+__device__ __forceinline__ const uint8_t* zero_run() { return reinterpret_cast<const uint8_t*>(g_hash_zeros); }
+__device__ __forceinline__ SegmentSource one_run(const uint8_t* p) { return {p, p, kFnvLaneBytes / 16}; }
+__device__ __forceinline__ SegmentSource two_runs(const Run& a, const Run& b, uint32_t ka) {
+    return {a.src ? a.src : zero_run(), (b.src ? b.src : zero_run()) - 16u * ka, ka};
+}
+__device__ __forceinline__ void load_source(const SegmentSource& f, uint32_t (&w)[kFnvLaneBytes / 4]) {
 #pragma unroll
     for (int k = 0; k < kFnvLaneBytes / 16; ++k) {
-        const bool in_a = uint32_t(k) < ka;
-        const uint8_t* q = in_a ? za + sa * uint64_t(k) : zb + sb * uint64_t(k - int(ka));
-        const u32x4 v = *(const gu32x4*) q;
+        const u32x4 v = *(const gu32x4*) ((uint32_t(k) < f.ka ? f.a : f.b) + 16 * k);
         w[4 * k] = v.x;
         w[4 * k + 1] = v.y;
         w[4 * k + 2] = v.z;
@@ -718,22 +732,12 @@ __device__ __forceinline__ void load_runs(const Run& a, const Run& b, uint32_t k
 }
 
 // A lane's whole segment inside extent X, where X holds the lane's whole wave and is wave-uniform (its fields stay in
-// scalar registers and no lane reads the extent table): a copy or the payload's own bytes in one run from one base, as
-// the plain hash loads, zeros without a load, pages in one run or two (across one page boundary).  False for a segment
-// over three pages or more (pages under 256 bytes), which the caller gathers chunk by chunk.
-__device__ __forceinline__ bool gather_in_extent(const HashExtent& X, uint8_t* base, uint64_t begin,
-                                                 uint32_t (&w)[kFnvLaneBytes / 4]) {
-    if (X.kind == kExtCopy) {
-        load_segment(X.src + (begin - X.off), w);
-        return true;
-    }
-    if (X.kind == kExtSelf) {
-        load_segment(base + begin, w);
-        return true;
-    }
-    if (X.kind == kExtZero) {
-#pragma unroll
-        for (int i = 0; i < kFnvLaneBytes / 4; ++i) w[i] = 0u;
+// scalar registers and no lane reads the extent table): a copy, the payload's own bytes or zeros in one run, pages in one
+// run or two (across one page boundary).  False for a segment over three pages or more (pages under 256 bytes), which the
+// caller gathers chunk by chunk.
+__device__ __forceinline__ bool gather_in_extent(const HashExtent& X, uint8_t* base, uint64_t begin, SegmentSource& from) {
+    if (X.kind != kExtPages) {
+        from = one_run(X.kind == kExtCopy ? X.src + (begin - X.off) : X.kind == kExtSelf ? base + begin : zero_run());
         return true;
     }
     const uint64_t seg_end = begin + kFnvLaneBytes;
@@ -745,37 +749,28 @@ __device__ __forceinline__ bool gather_in_extent(const HashExtent& X, uint8_t* b
         b = run_at(X, a.end, base + a.end);
         if (b.end < seg_end) return false;
     }
-    load_runs(a, b, ka, w);
+    from = two_runs(a, b, ka);
     return true;
 }
 
-// The lane's segment [begin, begin + len) gathered into w, walking the extent table from the workgroup's first extent
-// (a wave over an extent boundary, a workgroup over three extents or more, the payload's last wave).  A segment in one
-// run or two issues its 16 loads at once from one or two bases; a segment over three runs or more, and the payload's
-// last partial segment, goes chunk by chunk into the payload, which the lane then reads back (its own stores, after a
-// fence).  The payload is written by store_wave below (the last partial segment only here).
-__device__ __forceinline__ void gather_segment(const HashExtent* ext, bool store, uint8_t* base, uint32_t e_group, uint64_t begin,
-                                               uint64_t len, uint32_t (&w)[kFnvLaneBytes / 4]) {
+// The lane's segment [begin, begin + len), walking the extent table from the workgroup's first extent (a wave over an
+// extent boundary, a workgroup over three extents or more, the payload's last wave).  A segment in one run or two is
+// loaded from them; a segment over three runs or more, and the payload's last partial segment, goes chunk by chunk into
+// the payload, which the lane then reads back (its own stores, after a fence).  The payload is written by store_wave
+// below (the last partial segment only here; its chunks are hashed by the closing kernel).
+__device__ __forceinline__ SegmentSource gather_segment(const HashExtent* ext, uint8_t* base, uint32_t e_group, uint64_t begin,
+                                                        uint64_t len) {
     uint32_t e = e_group;
     while (ext[e].end <= begin) ++e;
     HashExtent x = ext[e];
-    uint8_t* dst = base + begin;   // `base` + o addresses payload byte o of this workgroup's segment
     const uint64_t seg_end = begin + len;
-    const Run a = run_at(x, begin, dst);
+    const Run a = run_at(x, begin, base + begin);
     if (len == kFnvLaneBytes) {
-        Run b = a;
-        uint32_t ka = kFnvLaneBytes / 16;   // chunks from run a
-        bool two = a.end >= seg_end;
-        if (!two) {
-            ka = uint32_t((a.end - begin) >> 4);
-            if (a.end >= x.end) x = ext[++e];
-            b = run_at(x, a.end, dst + 16u * ka);
-            two = b.end >= seg_end;
-        }
-        if (two) {
-            load_runs(a, b, ka, w);
-            return;
-        }
+        if (a.end >= seg_end) return two_runs(a, a, kFnvLaneBytes / 16);
+        const uint32_t ka = uint32_t((a.end - begin) >> 4);   // chunks from run a
+        if (a.end >= x.end) x = ext[++e];
+        const Run b = run_at(x, a.end, base + a.end);
+        if (b.end >= seg_end) return two_runs(a, b, ka);
         // three runs or more: walk from the workgroup's first extent again (the look-ahead above may have moved past
         // the extent holding `begin`)
         e = e_group;
@@ -788,10 +783,10 @@ __device__ __forceinline__ void gather_segment(const HashExtent* ext, bool store
         const Run r = run_at(x, o, base + o);
         const uint64_t o0 = o, end = r.end < seg_end ? r.end : seg_end;
         for (; o < end; o += 16)
-            if (r.store && store) put16(base + o, r.src ? *(const gu32x4*) (r.src + (o - o0)) : u32x4{0u, 0u, 0u, 0u});
+            if (r.store) put16(base + o, r.src ? *(const gu32x4*) (r.src + (o - o0)) : u32x4{0u, 0u, 0u, 0u});
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");   // the lane's stores complete before its reads
-    if (len == kFnvLaneBytes) load_segment(dst, w);
+    return one_run(len == kFnvLaneBytes ? base + begin : zero_run());
 }
 
 // The wave's 16 KiB of gathered payload into the payload with coalesced stores: each lane holds 256 contiguous bytes,
@@ -847,15 +842,20 @@ __global__ void __launch_bounds__(kFnvThreads) __attribute__((amdgpu_waves_per_e
     __shared__ u32x4 s_xpose[kMapped ? kFnvThreads / 64 : 1][8 * kXposeRow];
     __shared__ u32x4 s_weights[kWeightChunks];
     if (!kCarried && threadIdx.x == 0) L.ticket = atomicAdd(kernel_args()->ctl, 1u);
-    {
-        u32x4 weights[kWeightChunks / kFnvThreads];
-#pragma unroll
-        for (int i = 0; i < kWeightChunks / kFnvThreads; ++i)
-            weights[i] = ((const gu32x4*) &g_sum_weights.w[0][0][0])[i * kFnvThreads + threadIdx.x];
-#pragma unroll
-        for (int i = 0; i < kWeightChunks / kFnvThreads; ++i) s_weights[i * kFnvThreads + threadIdx.x] = weights[i];
-    }
+    // the sums' weights into LDS, by `threads` threads
+    const auto stage_weights = [&](uint32_t thread, uint32_t threads) {
+#pragma unroll 2
+        for (uint32_t i = thread; i < uint32_t(kWeightChunks); i += threads)
+            s_weights[i] = ((const gu32x4*) &g_sum_weights.w[0][0][0])[i];
+    };
+    if constexpr (kCarried) stage_weights(threadIdx.x, kFnvThreads);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint64_t share_end = 0;   // mapped: the end of the last extent of the lane's share of the map
+    if constexpr (kMapped) {
+        ConstArgs* a = kernel_args();
+        const uint32_t share = (a->map.n_ext + 63u) / 64u;
+        share_end = a->map.ext[min((threadIdx.x % 64u + 1u) * share, a->map.n_ext) - 1u].end;
+    }
     __syncthreads();
     uint64_t total = 0, total_part = 0;   // thread 0: the workgroup's sums
     uint32_t g = kCarried ? blockIdx.x : __builtin_amdgcn_readfirstlane(L.ticket);
@@ -873,10 +873,7 @@ __global__ void __launch_bounds__(kFnvThreads) __attribute__((amdgpu_waves_per_e
         const auto address_of = [&]() -> const uint8_t* {
             ConstArgs* a = kernel_args();
             const uint64_t begin = begin_of();
-            if (!a->map.seg) return a->data + begin;
-            // a payload read where its segments hold it: this workgroup's 64 KiB lie in segment k
-            const uint64_t k = uint64_t(g) * kFnvGroupBytes / a->map.seg_bytes;
-            return a->map.seg[k] + (begin - k * a->map.seg_bytes);
+            return (a->map.seg ? payload_base(g) : a->data) + begin;
         };
         const uint32_t len = bytes_of();
         const bool full = kMapped ? len != 0u : len == kFnvLaneBytes && kernel_args()->aligned;
@@ -895,41 +892,61 @@ __global__ void __launch_bounds__(kFnvThreads) __attribute__((amdgpu_waves_per_e
         uint32_t w[kFnvLaneBytes / 4] = {};
         uint8_t* base = nullptr;   // mapped: `base` + o addresses payload byte o in the segment holding this workgroup's bytes
         if constexpr (kMapped) {
-            // the workgroup's part of the map in one round trip: its 14 words read together through the constant address
-            // space (scalar loads; the map does not change during the launch) and held from here, rather than each field
-            // loaded in the branch that first needs it, one round trip after another
-            typedef const __attribute__((address_space(4))) uint64_t ConstWord;
+            // the extent holding the workgroup's first byte: every lane has read the end of the last extent of its share of
+            // the table while the ticket was on its way, so the ends at or before that byte count the shares before it
             ConstArgs* a = kernel_args();
-            const ConstWord* q = (const ConstWord*) (a->map.grp + g);
-            uint64_t h[14];
+            const uint64_t lo = uint64_t(g) * kFnvGroupBytes;
+            uint32_t first = uint32_t(__popcll(__ballot(share_end <= lo)));
+            const uint32_t share = (a->map.n_ext + 63u) / 64u;
+            if (share > 1) {   // then one by one inside that share, 64 at a time
+                first *= share;
+                for (uint32_t at = 0; at < share; at += 64) {
+                    const uint32_t i = min(first + uint32_t(lane), a->map.n_ext - 1u);
+                    const uint32_t before = uint32_t(__popcll(__ballot(a->map.ext[i].end <= lo)));
+                    first += before;
+                    if (before < 64) break;
+                }
+            }
+            first = min(first, a->map.n_ext - 1u);
+            // that extent and the next, read together through the constant address space (scalar loads; the map does not
+            // change during the launch, and consecutive workgroups read the same lines) and held from here
+            typedef const __attribute__((address_space(4))) uint64_t ConstWord;
+            const ConstWord* q0 = (const ConstWord*) (a->map.ext + first);
+            const ConstWord* q1 = (const ConstWord*) (a->map.ext + min(first + 1u, a->map.n_ext - 1u));
+            uint64_t h[12];
 #pragma unroll
-            for (int i = 0; i < 14; ++i) h[i] = q[i];
+            for (int i = 0; i < 6; ++i) h[i] = q0[i], h[6 + i] = q1[i];
+            base = payload_base(g);
             asm volatile("" ::"s"(h[0]), "s"(h[1]), "s"(h[2]), "s"(h[3]), "s"(h[4]), "s"(h[5]), "s"(h[6]), "s"(h[7]),
-                         "s"(h[8]), "s"(h[9]), "s"(h[10]), "s"(h[11]), "s"(h[12]), "s"(h[13]));
-            HashGroup hg;
-            static_assert(offsetof(HashGroup, pad) == 14 * 8, "the words read are the group's fields");
-            __builtin_memcpy(&hg, h, sizeof(h));
-            base = hg.base;
+                         "s"(h[8]), "s"(h[9]), "s"(h[10]), "s"(h[11]));
+            HashExtent x0, x1;
+            static_assert(sizeof(HashExtent) == 48, "the words read are the extent's fields");
+            __builtin_memcpy(&x0, h, 48);
+            __builtin_memcpy(&x1, h + 6, 48);
             const uint64_t begin = begin_of(), n_total = a->map.n_total;
+            SegmentSource from = one_run(zero_run());
             if (begin < n_total) {
                 const uint64_t wave_lo = (uint64_t(g) * kFnvThreads + uint64_t(wave) * 64) * kFnvLaneBytes;
                 const uint64_t wave_hi = wave_lo + 64u * kFnvLaneBytes;
                 bool done = false;
-                if (hg.two && wave_hi <= n_total) {   // every lane of the wave whole, inside one of the two extents
-                    if (wave_hi <= hg.x[0].end)
-                        done = gather_in_extent(hg.x[0], base, begin, w);
-                    else if (wave_lo >= hg.x[0].end)
-                        done = gather_in_extent(hg.x[1], base, begin, w);
+                if (wave_hi <= n_total) {   // every lane of the wave whole, inside one of the two extents
+                    if (wave_hi <= x0.end)
+                        done = gather_in_extent(x0, base, begin, from);
+                    else if (wave_lo >= x0.end && wave_hi <= x1.end)
+                        done = gather_in_extent(x1, base, begin, from);
                 }
                 if (!done) {
                     const uint64_t left = n_total - begin;
-                    gather_segment(a->map.ext, a->map.store, base, hg.first, begin,
-                                   left < kFnvLaneBytes ? left : kFnvLaneBytes, w);
+                    from = gather_segment(a->map.ext, base, first, begin, left < kFnvLaneBytes ? left : kFnvLaneBytes);
                 }
             }
+            load_source(from, w);
         } else if (full) {
             load_segment(address_of(), w);
         }
+        // every load is issued before the first word is used: paired as they come, the first two loads' words had the others
+        // wait for a memory round trip
+        __builtin_amdgcn_sched_barrier(0);
         pair_words(w);
 
         // the levels: every lane's map of the level (a whole segment from its two halves in registers, a partial or unaligned
@@ -957,15 +974,17 @@ __global__ void __launch_bounds__(kFnvThreads) __attribute__((amdgpu_waves_per_e
             level(Int<1>{}, Int<3>{}, Int<3>{}, 0, [] {});
             level(Int<2>{}, Int<6>{}, Int<2>{}, 0, [] {});
         } else {
-            level(Int<0>{}, Int<0>{}, Int<4>{}, kFirstSleeps, [] {});
+            // the waves that do not look back stage the weights meanwhile: before the ticket they spread the workgroups'
+            // starts, which every look-back then waits for
+            level(Int<0>{}, Int<0>{}, Int<4>{}, kFirstSleeps, [&] {
+                if (wave > 0) stage_weights(uint32_t(wave - 1) * 64u + uint32_t(lane), kFnvThreads - 64u);
+            });
             // the gathered payload is written while the last look-back waits (stores issued earlier meet the next
             // workgroups' gathers, later ones hold up the workgroup's end)
             level(Int<1>{}, Int<4>{}, Int<4>{}, kMapped ? kFirstSleepsMapped : kFirstSleeps, [&] {
                 if constexpr (kMapped) {
-                    ConstArgs* a = kernel_args();
-                    if (a->map.store)
-                        store_wave(s_xpose[wave], w, base, (uint64_t(g) * kFnvThreads + uint64_t(wave) * 64) * kFnvLaneBytes,
-                                   a->n, lane);
+                    store_wave(s_xpose[wave], w, base, (uint64_t(g) * kFnvThreads + uint64_t(wave) * 64) * kFnvLaneBytes,
+                               kernel_args()->n, lane);
                 }
             });
         }
@@ -1074,40 +1093,6 @@ hipError_t launch_fnv1a64(const void* data, uint64_t n, uint64_t seed, const uin
     // the finish reads the start state before it writes `out`, so `out` may be `seed_dev` itself
     hipLaunchKernelGGL(fnv_finish_kernel, dim3(1), dim3(1), 0, stream, ctl, seed, seed_dev, n, out, fault_out,
                        seed_dev != nullptr, expected, verdict, nullptr, 0u);
-    return hipGetLastError();
-}
-
-// Each hash workgroup's part of a map (HashGroup), one thread per workgroup: the extent holding the workgroup's first
-// byte (extents tile [0, bytes) in order, so the first whose end lies past it), that extent and the next, whether the
-// workgroup's bytes lie in those two, and where its segment puts payload byte 0.  Built on the device so that a map's
-// creation uploads its extents only (the parts are 128 bytes per 64 KiB: 6.4 MB for a 3.3 GB payload).
-__global__ void hash_groups_kernel(const HashExtent* ext, uint32_t n_ext, uint64_t bytes, uint8_t* const* segs,
-                                   uint32_t n_segs, uint64_t seg_bytes, HashGroup* grp, uint64_t groups) {
-    const uint64_t g = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (g >= groups) return;
-    const uint64_t o = g * uint64_t(kFnvGroupBytes), o_end = o + kFnvGroupBytes < bytes ? o + kFnvGroupBytes : bytes;
-    uint32_t lo = 0, hi = n_ext - 1;   // the first extent whose end lies past o (the last one at most)
-    while (lo < hi) {
-        const uint32_t mid = lo + (hi - lo) / 2;
-        if (ext[mid].end > o) hi = mid;
-        else lo = mid + 1;
-    }
-    HashGroup h{};
-    const uint64_t k = o / seg_bytes;
-    h.base = reinterpret_cast<uint8_t*>(reinterpret_cast<uintptr_t>(segs[k < n_segs ? k : n_segs - 1]) - k * seg_bytes);
-    h.first = lo;
-    h.x[0] = ext[lo];
-    if (lo + 1 < n_ext) h.x[1] = ext[lo + 1];
-    h.two = ext[lo].end >= o_end || (lo + 1 < n_ext && ext[lo + 1].end >= o_end) ? 1u : 0u;
-    grp[g] = h;
-}
-
-hipError_t launch_hash_groups(const HashExtent* ext, uint32_t n_ext, uint64_t bytes, uint8_t* const* segs,
-                              uint32_t n_segs, uint64_t seg_bytes, HashGroup* grp, uint64_t groups, hipStream_t stream) {
-    if (!groups) return hipSuccess;
-    if (!n_ext || !n_segs || !seg_bytes) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(hash_groups_kernel, dim3(unsigned((groups + 255) / 256)), dim3(256), 0, stream, ext, n_ext, bytes,
-                       segs, n_segs, seg_bytes, grp, groups);
     return hipGetLastError();
 }
 
