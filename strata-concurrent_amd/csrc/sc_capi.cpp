@@ -21,8 +21,7 @@
 #include "sc_internal.hpp"
 
 namespace sc {
-hipError_t launch_append(const AppendRows& rows, int n_rows, uint64_t tiles_per_row, const MoveGeo& geo, int32_t kind,
-                         hipStream_t stream);
+hipError_t launch_append(const AppendRows& rows, int n_rows, const MoveGeo& geo, int32_t kind, hipStream_t stream);
 hipError_t launch_move(const MoveRow* rows, const uint16_t* tile_row, const MoveGeo& geo, uint64_t n_tiles,
                        int64_t grid, int32_t mix, bool xcd, hipStream_t stream, const uint32_t* gate = nullptr);
 hipError_t launch_page_order(const OrderGroup* groups, int32_t n_groups, int64_t max_pages, uint32_t max_blocks,
@@ -1764,25 +1763,23 @@ int append_launch(int32_t kind, const float* K, const float* V, int64_t T, int64
         void* codes[2] = {a.k, a.v};
         uint16_t* scales[2] = {a.ks, a.vs};
         for (int kv = 0; kv < 2; ++kv) {
-            sc::MoveRow& r = rows.row[n++];
-            r.kind = kind;
+            sc::AppendRows::Row& r = rows.row[n++];
             r.src = reinterpret_cast<const uint8_t*>(srcs[kv]);
             r.dst = static_cast<uint8_t*>(codes[kv]);
             r.dst2 = reinterpret_cast<uint8_t*>(scales[kv]);
             r.table = a.table;
-            r.pos0 = pos0;
-            r.ld = std::numeric_limits<int64_t>::max();   // the reference bounds no page: the caller sized the pools
-            r.aux = int32_t(T);
-            r.n = units;
         }
     }
     const uint64_t per_tile = kind == sc::kKv32 ? sc::kTileChunks : sc::kQuantUnitsPerTile;
-    const uint64_t tiles = (rows.row[0].n + per_tile - 1) / per_tile;
+    rows.n = units;
+    rows.pos0 = pos0;
+    rows.tokens = int32_t(T);
+    rows.tiles = uint32_t((units + per_tile - 1) / per_tile);
     sc::MoveGeo geo{};
     geo.row_chunks = sc::make_fastdiv(uint32_t(D * 2 / 16));
     geo.heads = sc::make_fastdiv(uint32_t(H));
     geo.page_size = sc::make_fastdiv(uint32_t(page_size));
-    SC_HIP(sc::launch_append(rows, n, tiles, geo, kind, static_cast<hipStream_t>(stream)), "kv_append launch");
+    SC_HIP(sc::launch_append(rows, n, geo, kind, static_cast<hipStream_t>(stream)), "kv_append launch");
     return ok();
 }
 

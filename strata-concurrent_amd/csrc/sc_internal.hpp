@@ -174,10 +174,19 @@ struct BatchArgs {
 
 // The rows of one kv_append call (sc_kv_append_async, sc_kv_append_q4_async), carried in the kernel arguments
 // rather than a device table: K and V into the paged pool, into the host copy and into the staging pool.  Every row
-// is of one kind (kKv32, kKvQ8 or kKvQ4) and spans the same number of tiles.
+// is of one kind (kKv32, kKvQ8 or kKvQ4) and of one length, so a row is its pointers.
 constexpr int kAppendMaxRows = 6;
 struct AppendRows {
-    MoveRow row[kAppendMaxRows];
+    uint64_t n;        // chunks (kKv32) or (token, head) rows (quantized) of each row
+    int64_t pos0;
+    int32_t tokens;
+    uint32_t tiles;    // of each row
+    struct Row {
+        const uint8_t* src;
+        uint8_t* dst;
+        uint8_t* dst2;          // kKvQ8: the f16 scale pool
+        const int32_t* table;   // null: identity
+    } row[kAppendMaxRows];
 };
 
 // A paged slot parked into, or resumed from, a pinned host image by one kernel that writes or reads the mapped host

@@ -1157,58 +1157,52 @@ hipError_t launch_move(const MoveRow* rows, const uint16_t* tile_row, const Move
 // ---- kv_append: one call's rows in the kernel arguments -----------------------------------------------------------
 // The reference's per-layer prefill writers (kv_append, src/prefill/kernels.cu:558-625; kv_append_q4,
 // src/kernels/cuda/kv_q4.cu:111-135,205-215) take their destinations as arguments and allocate nothing, so this launch
-// takes its up to six rows the same way.  Row k owns tiles [k * tiles_per_row, (k + 1) * tiles_per_row); the switch
-// reads the selected row with scalar loads from the argument segment (an indexed read of the argument array would
-// copy it to scratch first).
+// takes its up to six rows the same way, one per blockIdx.y.  What bounds a call of a few tokens is latency: the kernel's
+// arguments lie in host memory, so the row's words are read together, as soon as its index is known, through the argument
+// segment with scalar loads (an indexed read of the argument array would copy it to scratch first), instead of after the
+// tile's row had been found by a 64-bit division of the two arguments before it (seven tokens appended to 12 int8 layers:
+// 49.5 us with the division, the row read after it).
 namespace {
 template <int kKind>
-__global__ void __launch_bounds__(kThreads) sc_append_kernel(AppendRows rows, int32_t n_rows, uint64_t tiles_per_row,
-                                                              MoveGeo geo) {
-    const uint64_t n_tiles = uint64_t(n_rows) * tiles_per_row;
-    for (uint64_t tile = blockIdx.x; tile < n_tiles; tile += gridDim.x) {
-        const int k = __builtin_amdgcn_readfirstlane(int(tile / tiles_per_row));
-        MoveRow r;
-        switch (k) {
-            case 0: r = rows.row[0]; break;
-            case 1: r = rows.row[1]; break;
-            case 2: r = rows.row[2]; break;
-            case 3: r = rows.row[3]; break;
-            case 4: r = rows.row[4]; break;
-            default: r = rows.row[5]; break;
-        }
-        const uint64_t local = tile - uint64_t(k) * tiles_per_row;
+__global__ void __launch_bounds__(kThreads) sc_append_kernel(AppendRows, MoveGeo geo) {
+    using karg = __attribute__((address_space(4))) const AppendRows*;
+    const karg args = (karg) __builtin_amdgcn_kernarg_segment_ptr();
+    MoveRow r{};
+    const auto& a = args->row[blockIdx.y];
+    r.src = a.src;
+    r.dst = a.dst;
+    r.dst2 = a.dst2;
+    r.table = a.table;
+    r.n = args->n;
+    r.pos0 = args->pos0;
+    r.aux = args->tokens;
+    r.ld = INT64_MAX;   // the reference bounds no page: the caller sized the pools
+    const uint32_t tiles = args->tiles;
+    for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
         if constexpr (kKind == kKv32) {
-            if (r.table) tile_kv32<true>(r, geo, local);
-            else tile_kv32<false>(r, geo, local);
+            if (r.table) tile_kv32<true>(r, geo, tile);
+            else tile_kv32<false>(r, geo, tile);
         } else if constexpr (kKind == kKvQ8) {
-            if (r.table) tile_q8<true>(r, geo, local);
-            else tile_q8<false>(r, geo, local);
+            if (r.table) tile_q8<true>(r, geo, tile);
+            else tile_q8<false>(r, geo, tile);
         } else {
-            tile_q4(r, geo, local);
+            tile_q4(r, geo, tile);
         }
     }
 }
 }  // namespace
 
-hipError_t launch_append(const AppendRows& rows, int n_rows, uint64_t tiles_per_row, const MoveGeo& geo, int32_t kind,
-                         hipStream_t stream) {
-    if (n_rows <= 0 || tiles_per_row == 0) return hipSuccess;
+hipError_t launch_append(const AppendRows& rows, int n_rows, const MoveGeo& geo, int32_t kind, hipStream_t stream) {
+    if (n_rows <= 0 || rows.tiles == 0) return hipSuccess;
     if (n_rows > kAppendMaxRows || (kind != kKv32 && kind != kKvQ8 && kind != kKvQ4)) return hipErrorInvalidValue;
-    const uint64_t n_tiles = uint64_t(n_rows) * tiles_per_row;
     // one workgroup per tile, as the plans launch (the 12 per-layer calls at 128K measured alike with 65536 workgroups
     // for f16 and 262144 for the quantizing rows: f16 1.636 against 1.640 ms, int8 1.409 against 1.410)
-    const uint64_t cap = uint64_t(1) << 20;
-    const dim3 blocks(unsigned(n_tiles < cap ? n_tiles : cap)), threads(kThreads);
+    const uint32_t cap = (1u << 20) / uint32_t(n_rows);
+    const dim3 blocks(rows.tiles < cap ? rows.tiles : cap, unsigned(n_rows)), threads(kThreads);
     switch (kind) {
-        case kKv32:
-            hipLaunchKernelGGL(sc_append_kernel<kKv32>, blocks, threads, 0, stream, rows, n_rows, tiles_per_row, geo);
-            break;
-        case kKvQ8:
-            hipLaunchKernelGGL(sc_append_kernel<kKvQ8>, blocks, threads, 0, stream, rows, n_rows, tiles_per_row, geo);
-            break;
-        default:
-            hipLaunchKernelGGL(sc_append_kernel<kKvQ4>, blocks, threads, 0, stream, rows, n_rows, tiles_per_row, geo);
-            break;
+        case kKv32: hipLaunchKernelGGL(sc_append_kernel<kKv32>, blocks, threads, 0, stream, rows, geo); break;
+        case kKvQ8: hipLaunchKernelGGL(sc_append_kernel<kKvQ8>, blocks, threads, 0, stream, rows, geo); break;
+        default: hipLaunchKernelGGL(sc_append_kernel<kKvQ4>, blocks, threads, 0, stream, rows, geo); break;
     }
     return hipGetLastError();
 }
