@@ -375,44 +375,79 @@ __device__ __forceinline__ uint64_t segment_sum(const uint8_t* p, uint64_t n, ui
     return acc * pow_prime(n - begin - len);
 }
 
-// h = seed * p^n + the sum of the workgroups' sums (mod 2^64; the order of the additions does not matter), `acc` being
-// that sum, or null for an empty input.  `fault` is the launch's fault word (null for an empty input, which has no
-// waits): a wait that ran out (kFaultWait) or carries that do not match the input (kFaultCarry) make h unusable, and the
-// launch says so at `fault_out` - the fault word, 0 for none, or, for a chained piece (`sticky`), or'ed into what the
-// earlier pieces left there, so a chain reports a fault of any of its pieces.  With `verdict`, also 1 there when h
-// equals `expected` and the launch has no fault, else 0: a later kernel on the stream can act on the check without a
-// host round trip.
-__global__ void fnv_finish_kernel(const uint32_t* ctl, uint64_t seed, const uint64_t* seed_dev, uint64_t n, uint64_t* out,
-                                  uint32_t* fault_out, bool sticky, uint64_t expected, uint32_t* verdict,
-                                  const uint8_t* tail, uint32_t tail_len) {
-    // the whole segments' sums are relative to the end of the last workgroup's 64 KiB
-    uint64_t h = start_state(seed, seed_dev) * pow_prime(n);
-    if (ctl) {
-        const uint64_t* acc = reinterpret_cast<const uint64_t*>(ctl + 2);
-        const uint64_t past = (kFnvGroupBytes - n % kFnvGroupBytes) % kFnvGroupBytes;
-        uint64_t back = 1, b = kPrimeInv;
-        for (uint64_t e = past; e; e >>= 1, b *= b)
-            if (e & 1) back *= b;
-        h += acc[0] * back + acc[1];
-    }
-    // the mapped hash leaves the payload's last partial lane segment (under 256 bytes, whole 16-byte chunks at a 16-byte
-    // aligned address) to this thread: its chunks are loaded at once, then hashed a byte at a time from registers
-    // (a loop of byte loads took 14 us, each load waiting on the one before)
-    if (tail_len) {
-        u32x4 c[kFnvLaneBytes / 16];
+// p^(2^k), p^(-2^k) and p^k.
+struct FinishPow {
+    uint64_t square[64], back[16], small[256];
+};
+constexpr FinishPow finish_pow() {
+    FinishPow t{};
+    uint64_t a = kFnvPrime, b = kPrimeInv, c = 1;
+    for (int k = 0; k < 64; ++k, a *= a) t.square[k] = a;
+    for (int k = 0; k < 16; ++k, b *= b) t.back[k] = b;
+    for (int k = 0; k < 256; ++k, c *= kFnvPrime) t.small[k] = c;
+    return t;
+}
+__constant__ FinishPow kFinishPow = finish_pow();
+
+// Closes a hash, one wave: h = seed * p^n + the sums of the workgroups (mod 2^64; the order of the additions does not
+// matter), continued over the `tail_len` bytes at `tail` (the last partial lane segment of an aligned input, under 256
+// bytes).  `ctl` holds the launch's sums and its fault word (null for an empty input): a wait that ran out (kFaultWait) or
+// carries that do not match the input (kFaultCarry) make h unusable, and the launch says so at `fault_out` - the fault
+// word, 0 for none, or, for a chained piece (`sticky`), or'ed into what the earlier pieces left there, so a chain reports
+// a fault of any of its pieces.  With `verdict`, also 1 there when h equals `expected` and the launch has no fault, else
+// 0: a later kernel on the stream can act on the check without a host round trip.
+// What bounds it is its chain of dependent operations, which every hash waits for: the powers are a product over the lanes,
+// one bit of the exponent each, and the tail is hashed as the lane segments are, four bytes a lane in two levels (one
+// thread doing both took 5-8 us, and a tail hashed by its lane in the one-pass kernel, a byte load at a time, longer).
+__global__ void __launch_bounds__(64) fnv_finish_kernel(const uint32_t* ctl, uint64_t seed, const uint64_t* seed_dev, uint64_t n,
+                                                        uint64_t* out, uint32_t* fault_out, bool sticky, uint64_t expected,
+                                                        uint32_t* verdict, const uint8_t* tail, uint32_t tail_len) {
+    const uint32_t lane = threadIdx.x;
+    // this lane's bytes of the tail
+    const uint32_t count = tail_len > 4u * lane ? min(tail_len - 4u * lane, 4u) : 0u;
+    uint32_t bytes[4];
 #pragma unroll
-        for (int k = 0; k < kFnvLaneBytes / 16; ++k)
-            c[k] = uint32_t(k) * 16u < tail_len ? *(const gu32x4*) (tail + 16 * k) : u32x4{0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int k = 0; k < kFnvLaneBytes / 16; ++k) {
-            if (uint32_t(k) * 16u >= tail_len) break;
-            const uint32_t word[4] = {c[k].x, c[k].y, c[k].z, c[k].w};
-#pragma unroll
-            for (int b = 0; b < 16; ++b)
-                if (uint32_t(k) * 16u + uint32_t(b) < tail_len) h = (h ^ ((word[b / 4] >> (8 * (b % 4))) & 0xFFu)) * kFnvPrime;
-        }
-    }
+    for (uint32_t i = 0; i < 4; ++i) bytes[i] = i < count ? tail[4u * lane + i] : 0u;
+    const uint64_t* acc = reinterpret_cast<const uint64_t*>(ctl + 2);
+    const uint64_t start = start_state(seed, seed_dev), whole = ctl ? acc[0] : 0u, part = ctl ? acc[1] : 0u;
     const uint32_t bad = ctl ? ctl[1] : 0u;   // kFaultWait and / or kFaultCarry
+    // the whole segments' sums are relative to the end of the last 64 KiB
+    const uint32_t past = uint32_t((kFnvGroupBytes - n % kFnvGroupBytes) % kFnvGroupBytes);
+    uint64_t pow_n = (n >> lane) & 1u ? kFinishPow.square[lane] : 1u;
+    uint64_t back = lane < 16u && ((past >> lane) & 1u) ? kFinishPow.back[lane] : 1u;
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) pow_n *= shfl_xor64(pow_n, m), back *= shfl_xor64(back, m);
+    uint64_t h = start * pow_n + whole * back + part;
+    if (tail_len) {
+        uint32_t low = 0;   // the true low byte at the lane's bytes, level by level
+        const auto level = [&](auto first_bit) {
+            constexpr int kJ = decltype(first_bit)::value;
+            uint32_t e[4], par = 0, at;
+#pragma unroll
+            for (uint32_t m = 0; m < 4; ++m) e[m] = low | (m << kJ);
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                par ^= bytes[i];
+#pragma unroll
+                for (uint32_t& x : e)
+                    if (i < count) x = __umul24((x ^ bytes[i]) & 0xFFu, kPrimeLow);
+            }
+            const uint32_t map = count ? map_of<kJ, 4>(e, par, count & 1u) : 0u;
+            (void) wave_apply<4>(map, (uint32_t(h) >> kJ) & 15u, at);
+            low |= at << kJ;
+        };
+        level(std::integral_constant<int, 0>{});
+        level(std::integral_constant<int, 4>{});
+        uint64_t sum = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i)
+            if (i < count) step_full(bytes[i], low, sum);
+        sum *= kFinishPow.small[count ? tail_len - 4u * lane - count : 0u];
+#pragma unroll
+        for (int m = 32; m > 0; m >>= 1) sum += shfl_xor64(sum, m);
+        h = h * kFinishPow.small[tail_len] + sum;
+    }
+    if (lane != 0) return;
     out[0] = h;
     if (fault_out) fault_out[0] = sticky ? (fault_out[0] | bad) : bad;
     if (verdict) verdict[0] = h == expected && !bad ? 1u : 0u;
@@ -458,7 +493,7 @@ template <int v>
 using Int = std::integral_constant<int, v>;
 struct OnepassArgs {
     const uint8_t* data;        // the input (16-byte aligned: `aligned`), or null with `map`
-    uint64_t n;                 // bytes hashed in the kernel
+    uint64_t n;                 // bytes hashed in the kernel: an aligned input's whole lane segments
     uint64_t seed;
     const uint64_t* seed_dev;
     uint32_t* ctl;              // [0] the ticket counter, [1] the fault word, [2..3], [4..5] the sums of whole and of partial segments
@@ -466,7 +501,8 @@ struct OnepassArgs {
     HashMapArgs map;
     FnvCarries carries;
     uint64_t carry_count;
-    uint32_t groups;            // workgroups' worth of input (64 KiB each)
+    uint32_t groups;            // workgroups' worth of input (64 KiB each), the tail that the closing kernel hashes included
+    uint32_t pieces;            // 64 KiB pieces of the n bytes hashed in the kernel
     uint32_t spin_limit;
     uint32_t aligned;
 };
@@ -887,7 +923,7 @@ __global__ void __launch_bounds__(kFnvThreads) __attribute__((amdgpu_waves_per_e
         }
         // what the workgroup's sum is worth where the last one ends; read here, with the data, rather than when the sum is
         // there and everything else done
-        const uint32_t rest = kernel_args()->groups - 1u - g;
+        const uint32_t rest = kernel_args()->pieces - 1u - g;   // (the tail's own workgroup sums nothing)
         const uint64_t worth = group_pow(0, rest) * group_pow(1, rest) * group_pow(2, rest) * group_pow(3, rest);
         uint32_t w[kFnvLaneBytes / 4] = {};
         uint8_t* base = nullptr;   // mapped: `base` + o addresses payload byte o in the segment holding this workgroup's bytes
@@ -1063,6 +1099,7 @@ uint32_t* enqueue_onepass(OnepassArgs a, uint8_t* workspace, uint64_t bytes, hip
     a.ctl = reinterpret_cast<uint32_t*>(workspace + w.off_ctl);
     a.status = reinterpret_cast<uint32_t*>(workspace + w.off_status);
     a.groups = uint32_t(w.groups);
+    a.pieces = uint32_t(fnv_workspace(a.n).groups);
     a.spin_limit = g_spin_limit.load();
     const uint64_t words = kStatusWords * w.groups, init_blocks = (words + kThreads - 1) / kThreads < 1024 ? (words + kThreads - 1) / kThreads : 1024;
     hipLaunchKernelGGL(fnv_onepass_init_kernel, dim3(unsigned(init_blocks)), dim3(kThreads), 0, stream, a.status, words, a.ctl);
@@ -1083,22 +1120,23 @@ hipError_t launch_fnv1a64(const void* data, uint64_t n, uint64_t seed, const uin
                           const FnvCarries& carries) {
     OnepassArgs a{};
     a.data = static_cast<const uint8_t*>(data);
-    a.n = n;
     a.aligned = (reinterpret_cast<uintptr_t>(data) & 15u) == 0;
+    a.n = a.aligned ? n & ~uint64_t(kFnvLaneBytes - 1) : n;
     a.seed = seed;
     a.seed_dev = seed_dev;
     a.carries = carries;
     a.carry_count = fnv_carry_count(n);
     const uint32_t* ctl = enqueue_onepass<false>(a, static_cast<uint8_t*>(workspace), n, stream);
     // the finish reads the start state before it writes `out`, so `out` may be `seed_dev` itself
-    hipLaunchKernelGGL(fnv_finish_kernel, dim3(1), dim3(1), 0, stream, ctl, seed, seed_dev, n, out, fault_out,
-                       seed_dev != nullptr, expected, verdict, nullptr, 0u);
+    hipLaunchKernelGGL(fnv_finish_kernel, dim3(1), dim3(64), 0, stream, ctl, seed, seed_dev, a.n, out, fault_out,
+                       seed_dev != nullptr, expected, verdict, a.data + a.n, uint32_t(n - a.n));
     return hipGetLastError();
 }
 
 // The gather fused with the hash: the payload's `map.n_total` bytes gathered into its segments and hashed, the whole
 // lane segments in the one-pass kernel and the last partial one (under 256 bytes, at `tail`) by the closing kernel,
-// which runs after every byte is in place.  With `verdict`, the closing kernel also leaves the check of the hash
+// which runs after every byte is in place.  A map that only reads is hashed by the plain kernel where its segments hold it.
+// With `verdict`, the closing kernel also leaves the check of the hash
 // against `expected` there, as sc_fnv1a64_check_async does.  The carries are those of the whole payload (`n_total`
 // bytes): a carry at a boundary inside the last partial lane segment cannot occur (boundaries are 64 KiB apart).
 hipError_t launch_fnv1a64_mapped(const HashMapArgs& map, const uint8_t* tail, uint64_t seed, uint64_t* out,
@@ -1113,12 +1151,10 @@ hipError_t launch_fnv1a64_mapped(const HashMapArgs& map, const uint8_t* tail, ui
     a.carries = carries;
     a.carry_count = fnv_carry_count(n_total);
     uint8_t* ws = static_cast<uint8_t*>(workspace);
-    // a map that only reads: the plain kernel hashes the payload where its segments hold it, the last partial lane segment
-    // included (no gather, so nothing waits for bytes to be placed)
-    a.n = map.store ? n_full : n_total;
+    a.n = n_full;
     const uint32_t* ctl = map.store ? enqueue_onepass<true>(a, ws, n_total, stream) : enqueue_onepass<false>(a, ws, n_total, stream);
-    hipLaunchKernelGGL(fnv_finish_kernel, dim3(1), dim3(1), 0, stream, ctl, seed, nullptr, a.n, out, fault_out, false, expected,
-                       verdict, map.store ? tail : nullptr, uint32_t(n_total - a.n));
+    hipLaunchKernelGGL(fnv_finish_kernel, dim3(1), dim3(64), 0, stream, ctl, seed, nullptr, n_full, out, fault_out, false,
+                       expected, verdict, tail, uint32_t(n_total - n_full));
     return hipGetLastError();
 }
 
