@@ -44,6 +44,7 @@
 #include <type_traits>
 
 #include "sc_handoff.h"
+#include "sc_hash_math.hpp"
 #include "sc_internal.hpp"
 
 namespace sc {
@@ -889,8 +890,7 @@ __global__ void __launch_bounds__(kFnvThreads) __attribute__((amdgpu_waves_per_e
     uint64_t share_end = 0;   // mapped: the end of the last extent of the lane's share of the map
     if constexpr (kMapped) {
         ConstArgs* a = kernel_args();
-        const uint32_t share = (a->map.n_ext + 63u) / 64u;
-        share_end = a->map.ext[min((threadIdx.x % 64u + 1u) * share, a->map.n_ext) - 1u].end;
+        share_end = a->map.ext[ExtentSpan{0u, a->map.n_ext}.sample(threadIdx.x % 64u)].end;
     }
     __syncthreads();
     uint64_t total = 0, total_part = 0;   // thread 0: the workgroup's sums
@@ -929,21 +929,13 @@ __global__ void __launch_bounds__(kFnvThreads) __attribute__((amdgpu_waves_per_e
         uint8_t* base = nullptr;   // mapped: `base` + o addresses payload byte o in the segment holding this workgroup's bytes
         if constexpr (kMapped) {
             // the extent holding the workgroup's first byte: every lane has read the end of the last extent of its share of
-            // the table while the ticket was on its way, so the ends at or before that byte count the shares before it
+            // the table while the ticket was on its way; a table of more than 64 is sampled again inside the share found
             ConstArgs* a = kernel_args();
             const uint64_t lo = uint64_t(g) * kFnvGroupBytes;
-            uint32_t first = uint32_t(__popcll(__ballot(share_end <= lo)));
-            const uint32_t share = (a->map.n_ext + 63u) / 64u;
-            if (share > 1) {   // then one by one inside that share, 64 at a time
-                first *= share;
-                for (uint32_t at = 0; at < share; at += 64) {
-                    const uint32_t i = min(first + uint32_t(lane), a->map.n_ext - 1u);
-                    const uint32_t before = uint32_t(__popcll(__ballot(a->map.ext[i].end <= lo)));
-                    first += before;
-                    if (before < 64) break;
-                }
-            }
-            first = min(first, a->map.n_ext - 1u);
+            ExtentSpan span{0u, a->map.n_ext};
+            span.narrow(uint32_t(__popcll(__ballot(share_end <= lo))));
+            while (span.size > 1u) span.narrow(uint32_t(__popcll(__ballot(a->map.ext[span.sample(uint32_t(lane))].end <= lo))));
+            const uint32_t first = span.first;
             // that extent and the next, read together through the constant address space (scalar loads; the map does not
             // change during the launch, and consecutive workgroups read the same lines) and held from here
             typedef const __attribute__((address_space(4))) uint64_t ConstWord;

@@ -1,6 +1,5 @@
 """The fused gather + hash over maps of many extents: each workgroup finds its first extent by sampling one end per share of
-the table and then looking inside that share, 64 ends at a time.  Table sizes around one share per lane, one look and two
-looks per share; extents of ragged lengths, some longer than a workgroup's 64 KiB, with gaps the map leaves as they are.
+the table and sampling again inside the share found.  Table sizes around one extent per share, one more sampling and two; extents of ragged lengths, some longer than a workgroup's 64 KiB, with gaps the map leaves as they are.
 Bytes and hash against numpy and the oracle's byte loop."""
 import numpy as np
 import pytest
@@ -8,7 +7,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("copies", [1, 2, 31, 32, 33, 63, 64, 65, 2048, 2080, 2200])
+@pytest.mark.parametrize("copies", [1, 2, 31, 32, 33, 63, 64, 65, 2048, 2080, 2200, 5000, 40000])
 def test_many_extents(sc, oracle, cuda, copies):
     rng = np.random.default_rng(copies)
     sizes = rng.integers(1, 60, copies) * 16
