@@ -306,7 +306,7 @@ OrderPlan order_plan(const std::vector<sc::MoveRow>& rows, const Geo& g) {
     }
     for (int& gi : o.row_group) gi = gi >= 0 ? keep[size_t(gi)] : -1;
     o.groups = std::move(kept);
-    for (sc::OrderGroup& G : o.groups) G.n_blocks = uint32_t((G.ld + sc::kOrderBlockPages - 1) / sc::kOrderBlockPages);
+    for (sc::OrderGroup& G : o.groups) G.n_blocks = sc::order_blocks(G.ld);
     // the order covers every page the tiles of its rows reach (whole tiles of whole pages)
     for (size_t k = 0; k < rows.size(); ++k) {
         if (o.row_group[k] < 0) continue;
@@ -1937,7 +1937,7 @@ int sc_plan_resume_append(const sc_geometry* g, const sc_batch_desc* d, sc_plan*
         p->payload = 0;   // depends on the device-resident lengths
         // workspace: [slots][ok][arena order group][inv][order pairs][counts]
         auto up = [](uint64_t x) { return (x + 255) / 256 * 256; };
-        const uint32_t n_blocks = uint32_t((uint64_t(d->arena_pages) + sc::kOrderBlockPages - 1) / sc::kOrderBlockPages);
+        const uint32_t n_blocks = sc::order_blocks(d->arena_pages);
         const uint64_t at_ok = up(sizeof(sc::BatchSlot) * sc::kMaxBatchSlots), at_group = at_ok + 256,
                        at_inv = at_group + up(sizeof(sc::OrderGroup)), at_order = at_inv + up(uint64_t(d->arena_pages) * 4),
                        at_counts = at_order + up(2 * order_len * 4), ws_bytes = at_counts + up(uint64_t(n_blocks) * 4);

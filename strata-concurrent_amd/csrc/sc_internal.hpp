@@ -105,12 +105,18 @@ static_assert(sizeof(MoveRow) == 80, "handoff table rows are 80 bytes");
 // writes one ascending run and scatters the reads instead, which this part takes better with non-temporal stores
 // (a 3.3 GB copy of permuted 4 KiB pages measured 64% of HBM peak in source order, 67.5-68% in destination order).
 // The order of one page table is rebuilt before every launch, since the table may change between launches: the
-// inverse table (physical page -> logical page) is scattered into `inv`, each block of kOrderBlockPages physical
+// inverse table (physical page -> logical page) is scattered into `inv`, each block of order_block_pages physical
 // pages counts its entries, and each block then writes its logical pages, ascending, after those of the blocks
 // before it, and clears its part of `inv` for the next launch.
-// 1024 pages a block: the counts and the lists of 32K-token tables took 4.8 and 4.9 us, against 7.6 and 9.5 us with 4096 (two
-// blocks a table leave most of the chip idle and each thread a chain of sixteen).
-constexpr int kOrderBlockPages = 1024;
+// Blocks of 1024 pages up to a pool of 2^22: the counts and the lists of 32K-token tables took 4.8 and 4.9 us, against 7.6
+// and 9.5 us with 4096 (two blocks a table leave most of the chip idle and each thread a chain of sixteen).  Past it 4096:
+// each block sums the counts of all before it, which passes the pool's own reading.  Carves of 1/8 of the pool's pages of
+// 128 bytes through one table: 2^22 pages 149 us with 1024 against 154 with 4096, 2^23 170 against 163, 2^25 745 against
+// 630; through twelve tables 2^20 225 against 233, 2^22 907 either way, 6 * 2^20 1515 against 1505, 2^24 4479 against 4123.
+constexpr int64_t kOrderSmallPool = int64_t(1) << 22;
+constexpr int kOrderSmallBlock = 1024, kOrderLargeBlock = 4096;
+constexpr int order_block_pages(int64_t ld) { return ld <= kOrderSmallPool ? kOrderSmallBlock : kOrderLargeBlock; }
+constexpr uint32_t order_blocks(int64_t ld) { return uint32_t((ld + order_block_pages(ld) - 1) / order_block_pages(ld)); }
 struct OrderGroup {
     const int32_t* table;   // logical page -> physical page
     int32_t* inv;           // [ld] physical page -> logical page; -1 between launches

@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "sc_arith.hpp"
 #include "sc_convert.hpp"
@@ -919,6 +920,8 @@ __global__ void ring_table_kernel(int32_t* table, int64_t n_blocks, int64_t n_sl
 
 // ---- destination order: the pre-pass of a plan whose rows write through page tables ------------------------------
 // (OrderGroup, sc_internal.hpp.)  Three launches, one group (page table) per blockIdx.y.
+template <int v>
+using Int = std::integral_constant<int, v>;
 
 // The inverse table: inv[table[lp]] = lp for the group's logical pages whose physical page is in the pool.
 __global__ void __launch_bounds__(kThreads) order_scatter_kernel(const OrderGroup* __restrict__ groups) {
@@ -950,15 +953,19 @@ __device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t& total) {
     return before + x - v;
 }
 
-// Entries per block of kOrderBlockPages physical pages.
+// Entries per block of order_block_pages physical pages.
 __global__ void __launch_bounds__(kThreads) order_count_kernel(const OrderGroup* __restrict__ groups) {
     const OrderGroup& G = groups[blockIdx.y];
     const uint32_t b = blockIdx.x;
     if (b >= G.n_blocks) return;
-    const int64_t base = int64_t(b) * kOrderBlockPages;
-    uint32_t c = 0;
-    for (int k = threadIdx.x; k < kOrderBlockPages; k += kThreads)
-        if (base + k < G.ld && G.inv[base + k] >= 0) ++c;
+    const auto count = [&](auto pages) {
+        const int64_t base = int64_t(b) * pages;
+        uint32_t c = 0;
+        for (int k = threadIdx.x; k < pages; k += kThreads)
+            if (base + k < G.ld && G.inv[base + k] >= 0) ++c;
+        return c;
+    };
+    const uint32_t c = order_block_pages(G.ld) == kOrderSmallBlock ? count(Int<kOrderSmallBlock>{}) : count(Int<kOrderLargeBlock>{});
     uint32_t total;
     (void) block_scan(c, total);
     if (threadIdx.x == 0) G.counts[b] = total;
@@ -967,7 +974,6 @@ __global__ void __launch_bounds__(kThreads) order_count_kernel(const OrderGroup*
 // Each block sums the counts before it, writes its entries, ascending by physical page, at that prefix and clears them
 // from inv; the last block fills the list past the last entry with -1.
 __global__ void __launch_bounds__(kThreads) order_write_kernel(const OrderGroup* __restrict__ groups) {
-    constexpr int kPer = kOrderBlockPages / kThreads;
     const OrderGroup& G = groups[blockIdx.y];
     const uint32_t b = blockIdx.x;
     if (b >= G.n_blocks) return;
@@ -975,25 +981,30 @@ __global__ void __launch_bounds__(kThreads) order_write_kernel(const OrderGroup*
     for (uint32_t i = threadIdx.x; i < b; i += kThreads) before += G.counts[i];
     uint32_t prefix;
     (void) block_scan(before, prefix);
-    const int64_t base = int64_t(b) * kOrderBlockPages + int64_t(threadIdx.x) * kPer;
-    int32_t e[kPer];
-    uint32_t c = 0;
-#pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-        e[k] = base + k < G.ld ? G.inv[base + k] : -1;
-        c += e[k] >= 0 ? 1u : 0u;
-    }
-    uint32_t total;
-    uint32_t at = prefix + block_scan(c, total);
     const uint32_t width = G.pairs ? 2u : 1u;
+    const auto write = [&](auto pages) {
+        constexpr int kPer = decltype(pages)::value / kThreads;
+        const int64_t base = int64_t(b) * pages + int64_t(threadIdx.x) * kPer;
+        int32_t e[kPer];
+        uint32_t c = 0;
 #pragma unroll
-    for (int k = 0; k < kPer; ++k)
-        if (e[k] >= 0) {
-            G.order[uint64_t(at) * width] = e[k];
-            if (G.pairs) G.order[uint64_t(at) * width + 1] = int32_t(base + k);
-            ++at;
-            G.inv[base + k] = -1;
+        for (int k = 0; k < kPer; ++k) {
+            e[k] = base + k < G.ld ? G.inv[base + k] : -1;
+            c += e[k] >= 0 ? 1u : 0u;
         }
+        uint32_t total;
+        uint32_t at = prefix + block_scan(c, total);
+#pragma unroll
+        for (int k = 0; k < kPer; ++k)
+            if (e[k] >= 0) {
+                G.order[uint64_t(at) * width] = e[k];
+                if (G.pairs) G.order[uint64_t(at) * width + 1] = int32_t(base + k);
+                ++at;
+                G.inv[base + k] = -1;
+            }
+        return total;
+    };
+    const uint32_t total = order_block_pages(G.ld) == kOrderSmallBlock ? write(Int<kOrderSmallBlock>{}) : write(Int<kOrderLargeBlock>{});
     if (b + 1 == G.n_blocks)
         for (uint64_t i = (uint64_t(prefix) + total) * width + threadIdx.x; i < G.order_len * width; i += kThreads)
             G.order[i] = -1;

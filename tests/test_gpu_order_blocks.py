@@ -1,5 +1,6 @@
-"""The destination order's list is counted and written in blocks of 1024 physical pages: pools that end one page before, on
-and one page after a block's end, and tables spread over several blocks, place every byte as the oracle does."""
+"""The destination order's list is counted and written in blocks of 1024 physical pages (4096 of a pool past 2^22): pools
+that end one page before, on and one page after a block's end, and tables spread over several blocks, place every byte as
+the oracle does."""
 import numpy as np
 import pytest
 
@@ -43,4 +44,28 @@ def test_order_at_the_blocks_edges(sc, oracle, cuda, n_pages, T):
             want = np.full(n_pages * H * ps * D, 0xEEEE, dtype=np.uint16)
             oracle.kv_append(inputs[kv][j], T, 0, tables[j], n_pages, H, D, ps, want)
             assert np.array_equal(got[f"{kv}{j}"].reshape(-1), want), f"{kv}{j} differs"
+    plan.destroy()
+
+
+@pytest.mark.parametrize("n_pages", [(1 << 22) - 1, 1 << 22, (1 << 22) + 1, (1 << 22) + 4096, (1 << 22) + 4097])
+def test_order_of_a_large_pool(sc, cuda, n_pages):
+    """Pools past 2^22 pages are counted and written in blocks of 4096 pages."""
+    T = n_pages // 8 + 1
+    print(f"case order of a large pool, pages={n_pages} T={T}", flush=True)
+    geo = sc.geometry(**{**GEO, "n_layers": 4, "n_head_kv": 1, "head_dim": 8, "page_size": 1})
+    table = np.random.default_rng(n_pages).permutation(n_pages)[:T].astype(np.int32)
+    table[T // 2] = n_pages - 1 if n_pages - 1 not in table else table[T // 2]
+    case = synth.SyntheticCase(geo, tokens=T, seed=n_pages)
+    slot = sc.new_slot(geo, T, n_pages=n_pages, tables=sc.device_tables([table]), fill=0xEE)
+    sc.device_sync()
+    plan = sc.plan_carve(geo, case.prefill, slot, with_gdn=False)
+    assert plan.order_groups == 1
+    for _ in range(2):
+        plan.launch()
+    sc.device_sync()
+    inputs, got = case.host_inputs(), slot.host_state()
+    for kv in ("k", "v"):
+        want = np.full((n_pages, 8), 0xEEEE, dtype=np.uint16)
+        want[table] = inputs[kv][0].reshape(T, 8)
+        assert np.array_equal(got[f"{kv}0"].reshape(n_pages, 8), want), f"{kv} differs"
     plan.destroy()
