@@ -1175,8 +1175,8 @@ hipError_t launch_move(const MoveRow* rows, const uint16_t* tile_row, const Move
 // tile's row had been found by a 64-bit division of the two arguments before it (seven tokens appended to 12 int8 layers:
 // 49.5 us with the division, the row read after it).
 namespace {
-template <int kKind>
-__global__ void __launch_bounds__(kThreads) sc_append_kernel(AppendRows, MoveGeo geo) {
+template <int kKind, int kWaves>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, kWaves))) sc_append_kernel(AppendRows, MoveGeo geo) {
     using karg = __attribute__((address_space(4))) const AppendRows*;
     const karg args = (karg) __builtin_amdgcn_kernarg_segment_ptr();
     MoveRow r{};
@@ -1211,11 +1211,17 @@ hipError_t launch_append(const AppendRows& rows, int n_rows, const MoveGeo& geo,
     // for f16 and 262144 for the quantizing rows: f16 1.636 against 1.640 ms, int8 1.409 against 1.410)
     const uint32_t cap = (1u << 20) / uint32_t(n_rows);
     const dim3 blocks(rows.tiles < cap ? rows.tiles : cap, unsigned(n_rows)), threads(kThreads);
-    switch (kind) {
-        case kKv32: hipLaunchKernelGGL(sc_append_kernel<kKv32>, blocks, threads, 0, stream, rows, geo); break;
-        case kKvQ8: hipLaunchKernelGGL(sc_append_kernel<kKvQ8>, blocks, threads, 0, stream, rows, geo); break;
-        default: hipLaunchKernelGGL(sc_append_kernel<kKvQ4>, blocks, threads, 0, stream, rows, geo); break;
-    }
+    // Long calls keep fewer waves on a SIMD: eight (up from seven, as the row's registers went) spread a call that passes
+    // the memory-side cache over more of memory at once.  Through page tables f16 rows of 131072 tokens took 143.2 us with
+    // eight and 140.7 with six (141.2 with seven, the row found by a division), int8 rows 129.6 with eight and 125.2 with
+    // five (127.9), q4_0 rows 117.7 and 117.0 (not worth an instance).  Below the lines eight are as fast or faster: f16
+    // rows of 8192 tokens 9.4 us against 10.1, int8 rows of 49152 tokens 37.8 against 38.9.
+    const uint64_t tiles = uint64_t(rows.tiles) * uint32_t(n_rows);
+    if (kind == kKv32 && tiles >= 8192) hipLaunchKernelGGL((sc_append_kernel<kKv32, 6>), blocks, threads, 0, stream, rows, geo);
+    else if (kind == kKv32) hipLaunchKernelGGL((sc_append_kernel<kKv32, 8>), blocks, threads, 0, stream, rows, geo);
+    else if (kind == kKvQ8 && tiles >= 16384) hipLaunchKernelGGL((sc_append_kernel<kKvQ8, 5>), blocks, threads, 0, stream, rows, geo);
+    else if (kind == kKvQ8) hipLaunchKernelGGL((sc_append_kernel<kKvQ8, 8>), blocks, threads, 0, stream, rows, geo);
+    else hipLaunchKernelGGL((sc_append_kernel<kKvQ4, 8>), blocks, threads, 0, stream, rows, geo);
     return hipGetLastError();
 }
 

@@ -217,3 +217,26 @@ def test_refusals_write_nothing(sc, cuda):
     for p in (pool, q8, q4):
         for b in p.values():
             assert (_read(sc, b) == SENTINEL).all()
+
+
+@pytest.mark.parametrize("fmt,T", [("f16", 32760), ("f16", 32768), ("f16", 32771), ("int8", 65528), ("int8", 65536),
+                                   ("int8", 65541)])
+def test_long_calls_match_oracle(sc, oracle, cuda, fmt, T):
+    """Calls at both sides of the tile counts from which a kernel instance of fewer waves takes them."""
+    print(f"case long kv_append {fmt} T={T}", flush=True)
+    pos0 = 3
+    n_logical = (pos0 + T + PS - 1) // PS
+    n_pages = n_logical + 3
+    x = _source(T, T)
+    K = sc.DeviceBuffer(x.size, "float32")
+    K.upload(x)
+    table = _table("holes", n_logical, n_pages)
+    tab = sc.DeviceBuffer(table.size, "int32")
+    tab.upload(table)
+    pool = _pools(sc, fmt, n_pages, host=False)
+    assert _append(sc, fmt, K.ptr, K.ptr, T, pos0, tab.ptr, pool) == 0, sc.last_error()
+    want_codes, want_scales = _expected(oracle, fmt, x, T, pos0, table, n_pages)
+    for kv in ("k", "v"):
+        assert np.array_equal(_read(sc, pool[kv]), want_codes), kv
+        if want_scales is not None:
+            assert np.array_equal(_read(sc, pool[kv + "s"]), want_scales), kv
