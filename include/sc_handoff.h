@@ -462,7 +462,7 @@ uint64_t sc_kv_block_bytes(int64_t n_head_kv, int64_t head_dim, int64_t page_siz
  * state is resolved a few bit planes at a time by xor prefixes and a look-back across workgroups, after which the hash
  * is a sum of independent per-segment terms.  The reference seeds every call with 1469598103934665603
  * (conversation_wire.hpp:196). */
-/* Device workspace the asynchronous form needs for `bytes` bytes of input (about bytes / 3000, at least 512 bytes). */
+/* Device workspace the asynchronous form needs for `bytes` bytes of input (about bytes / 8192, at least 256 bytes). */
 uint64_t sc_fnv1a64_workspace_bytes(uint64_t bytes);
 /* Enqueue the hash on `stream`; the result lands as one u64 at `out`, and the launch's status as one u32 at `fault`:
  * 0, or 1 when one of the kernel's bounded look-back waits ran out (never in a correct launch on a GPU that runs its

@@ -1070,7 +1070,7 @@ __global__ void __launch_bounds__(kThreads) fnv_onepass_init_kernel(uint32_t* st
 // The bound on each look-back wait, in window reads; tests lower it to force a wait to run out.
 std::atomic<uint32_t> g_spin_limit{kSpinLimit};
 
-// Workspace: [ticket, fault and sum words][status words: up to three per workgroup].
+// Workspace: [ticket, fault and sum words][status words: kStatusWords per workgroup].
 FnvWorkspace fnv_workspace(uint64_t n) {
     FnvWorkspace w{};
     w.segments = (n + kFnvLaneBytes - 1) / kFnvLaneBytes;
@@ -1078,7 +1078,7 @@ FnvWorkspace fnv_workspace(uint64_t n) {
     auto up = [](uint64_t x) { return (x + 255) / 256 * 256; };
     w.off_ctl = 0;
     w.off_status = 256;
-    w.bytes = w.off_status + 3 * up(w.groups * 4);
+    w.bytes = w.off_status + up(kStatusWords * 4 * w.groups);
     return w;
 }
 
@@ -1155,7 +1155,7 @@ hipError_t launch_fnv1a64_mapped(const HashMapArgs& map, const uint8_t* tail, ui
 // ---- the hash that allocates nothing ----------------------------------------------------------------------------------
 // For callers that cannot allocate (code under HIP graph capture, tight serving loops): the workspace is `scratch`, one
 // array per GPU that the library holds until the process ends, sized for inputs of up to SC_FNV_NOALLOC_MAX_BYTES
-// (fnv_workspace(4 GiB) is 0.75 MiB).  Every call clears all of it that it uses (the ticket, the fault word, the sum
+// (fnv_workspace(4 GiB) is 0.5 MiB).  Every call clears all of it that it uses (the ticket, the fault word, the sum
 // and the look-back's status words) with a kernel of its own before the hash kernel; a call after another on the same
 // stream is ordered after it, and calls that overlap on one GPU (on different streams) race on the one array.
 namespace {

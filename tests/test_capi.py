@@ -213,3 +213,10 @@ def test_kv_block_bytes_per_format(sc):
         assert sc.lib.sc_kv_block_bytes(heads, dim, ps, 0) == rows * dim * 2 * 2
         assert sc.lib.sc_kv_block_bytes(heads, dim, ps, 1) == rows * (dim + dim // 64 * 2) * 2
         assert sc.lib.sc_kv_block_bytes(heads, dim, ps, 2) == rows * (dim // 32 * 18) * 2
+
+
+def test_hash_workspace_holds_the_launch_words_only(sc):
+    """256 bytes of ticket, fault and sums, then two look-back words per 64 KiB, rounded to 256 bytes."""
+    for n in (0, 1, 65536, 65537, 32 << 16, (32 << 16) + 1, 3 << 30, 1 << 46):
+        groups = -(-n // 65536)
+        assert sc.lib.sc_fnv1a64_workspace_bytes(n) == 256 + -(-8 * groups // 256) * 256, n
