@@ -1,13 +1,13 @@
-"""The arithmetic the device FNV-1a's levels rest on (strata-concurrent_amd/csrc/sc_hash.hip), checked on the CPU
-against brute force: the low byte of the FNV-1a state is the machine l' = ((l ^ b) * 179) mod 256, and a level's
-map of a run of bytes says where the level's bits go given the true lower bits.
+"""The derivation the device FNV-1a's levels rest on, checked on the CPU against brute force: the low byte of the FNV-1a
+state is the machine l' = ((l ^ b) * 179) mod 256, and a level's map of a run of bytes says where the level's bits go
+given the true lower bits.
 
-The kernel computes a k-bit level's map from 2^(k-2) machine runs plus the byte parities of the run (the top two
-bits' terms follow from the term of the bit below and the parity of that bit), runs each 256-byte lane segment as two
-128-byte halves side by side, takes the lane's map as the second half's after the first's, and gets the bits at the
-midpoint by applying the first half's map to the start bits.  Each of these steps is restated here the way the kernel
-does it and compared with running the machine from every start value, so a wrong parity bit, a swapped composition
-order or a wrong midpoint fails.  The device kernel itself is compared with the byte loop in tests/test_gpu_hash.py.
+A k-bit level's map follows from 2^(k-2) machine runs plus the byte parities of the run (the top two bits' terms follow
+from the term of the bit below and the parity of that bit), a 256-byte segment's from its two 128-byte halves' (the second
+after the first), and the bits at the midpoint from the first half's map.  Each of these is restated here, for levels of
+two and three bits, and compared with running the machine from every start value.  These are checks of the mathematics:
+the kernel's own functions are compiled and compared with the byte loop in tests/test_hash_math.py, and the kernel itself
+in tests/test_gpu_hash.py.
 """
 import numpy as np
 import pytest
@@ -35,7 +35,7 @@ def brute_map(low, j, k, data):
 
 
 def shortcut_map(low, j, k, data):
-    """The kernel's form (map3_of / map2_of): 2^(k-2) machines, the rest from the byte parities."""
+    """2^(k-2) machines, the rest from the byte parities."""
     par = 0
     for b in data:
         par ^= int(b)
@@ -61,7 +61,7 @@ def map_w(m, a, c):
 
 
 def compose(k, g, f):
-    """g after f, as compose<k> in the kernel."""
+    """g after f."""
     tf = f & 1
     r = tf ^ (g & 1)
     for a in (0, 1):
@@ -114,9 +114,9 @@ def test_the_parity_term_matters():
 
 
 def test_halves_compose_to_the_segment_and_give_the_midpoint():
-    """A 256-byte segment as two 128-byte halves, level by level, as the kernel's level1/2/3_maps and the kernel body:
-    the lane's map is the second half's after the first's, and the first half's map applied to the true start bits
-    gives the bits at the midpoint, where the next level's second-half machines start."""
+    """A 256-byte segment as two 128-byte halves, level by level: the segment's map is the second half's after the first's,
+    and the first half's map applied to the true start bits gives the bits at the midpoint, where the next level's
+    second-half machines start."""
     rng = np.random.default_rng(31)
     for trial in range(600):
         seg = rng.integers(0, 256, 256)

@@ -1,5 +1,6 @@
-"""The arithmetic of the device FNV-1a's four-bit levels and of its sums on the matrix cores
-(strata-concurrent_amd/csrc/sc_hash.hip), restated on the CPU and compared with the byte loop."""
+"""The derivation of the device FNV-1a's four-bit levels and of its sums on the matrix cores, restated on the CPU and compared
+with the byte loop.  These are checks of the mathematics: the kernel's own functions and tables are compiled and compared
+with the byte loop in tests/test_hash_math.py."""
 import numpy as np
 import pytest
 
@@ -15,7 +16,7 @@ def run(l, data):
 
 
 def map_of(low, j, k, data):
-    """map_of in the kernel: 2^(k-2) machines, the top bit's terms for a set bit below it from the byte parities."""
+    """2^(k-2) machines, the top bit's terms for a set bit below it from the byte parities."""
     ends = [run(low | (m << j), data) for m in range(1 << (k - 2))]
     flip = ((int(np.bitwise_xor.reduce(data)) if len(data) else 0) >> (j + k - 2) & 1) ^ (len(data) & 1)
     out = 0
@@ -66,7 +67,7 @@ def test_level_maps_take_every_start_to_its_end(j, k):
 
 
 def test_wave_maps_by_counting_lower_lanes():
-    """wave_apply in the kernel: 64 lanes' maps from a start state, each bit by the parity of the lower lanes' terms."""
+    """64 lanes' maps from a start state, each bit by the parity of the lower lanes' terms."""
     rng = np.random.default_rng(3)
     for k in (2, 3, 4):
         for st in range(1 << k):
