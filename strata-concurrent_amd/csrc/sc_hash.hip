@@ -710,10 +710,14 @@ __global__ void __launch_bounds__(kFnvThreads) __attribute__((amdgpu_waves_per_e
     };
     if constexpr (kCarried) stage_weights(threadIdx.x, kFnvThreads);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    uint64_t share_end = 0;   // mapped: the end of the last extent of the lane's share of the map
+    // mapped: the table of extents, and the end of the last extent of the lane's share of it
+    const HashExtent* ext = nullptr;
+    uint32_t n_ext = 0;
+    uint64_t share_end = 0;
     if constexpr (kMapped) {
         ConstArgs* a = kernel_args();
-        share_end = a->map.ext[ExtentSpan{0u, a->map.n_ext}.sample(threadIdx.x % 64u)].end;
+        ext = a->map.ext, n_ext = a->map.n_ext;
+        share_end = ext[ExtentSpan{0u, n_ext}.sample(threadIdx.x % 64u)].end;
     }
     __syncthreads();
     uint64_t total = 0, total_part = 0;   // thread 0: the workgroup's sums
@@ -745,9 +749,14 @@ __global__ void __launch_bounds__(kFnvThreads) __attribute__((amdgpu_waves_per_e
             after = g < a->carry_count ? uint32_t(a->carries.in[g]) : 0x100u;
         }
         // what the workgroup's sum is worth where the last one ends; read here, with the data, rather than when the sum is
-        // there and everything else done
-        const uint32_t rest = kernel_args()->pieces - 1u - g;   // (the tail's own workgroup sums nothing)
-        const uint64_t worth = group_pow(0, rest) * group_pow(1, rest) * group_pow(2, rest) * group_pow(3, rest);
+        // there and everything else done (mapped: once the loads' sources are found, which these reads would hold up: the
+        // 128K capture + hash 1.776 against 1.789 ms; the plain hash the other way, 1.344 against 1.348)
+        uint64_t worth = 0;
+        const auto read_worth = [&] {
+            const uint32_t rest = kernel_args()->pieces - 1u - g;   // (the tail's own workgroup sums nothing)
+            worth = group_pow(0, rest) * group_pow(1, rest) * group_pow(2, rest) * group_pow(3, rest);
+        };
+        if constexpr (!kMapped) read_worth();
         uint32_t w[kFnvLaneBytes / 4] = {};
         uint8_t* base = nullptr;   // mapped: `base` + o addresses payload byte o in the segment holding this workgroup's bytes
         if constexpr (kMapped) {
@@ -755,15 +764,15 @@ __global__ void __launch_bounds__(kFnvThreads) __attribute__((amdgpu_waves_per_e
             // the table while the ticket was on its way; a table of more than 64 is sampled again inside the share found
             ConstArgs* a = kernel_args();
             const uint64_t lo = uint64_t(g) * kFnvGroupBytes;
-            ExtentSpan span{0u, a->map.n_ext};
+            ExtentSpan span{0u, n_ext};
             span.narrow(uint32_t(__popcll(__ballot(share_end <= lo))));
-            while (span.size > 1u) span.narrow(uint32_t(__popcll(__ballot(a->map.ext[span.sample(uint32_t(lane))].end <= lo))));
+            while (span.size > 1u) span.narrow(uint32_t(__popcll(__ballot(ext[span.sample(uint32_t(lane))].end <= lo))));
             const uint32_t first = span.first;
             // that extent and the next, read together through the constant address space (scalar loads; the map does not
             // change during the launch, and consecutive workgroups read the same lines) and held from here
             typedef const __attribute__((address_space(4))) uint64_t ConstWord;
-            const ConstWord* q0 = (const ConstWord*) (a->map.ext + first);
-            const ConstWord* q1 = (const ConstWord*) (a->map.ext + min(first + 1u, a->map.n_ext - 1u));
+            const ConstWord* q0 = (const ConstWord*) (ext + first);
+            const ConstWord* q1 = (const ConstWord*) (ext + min(first + 1u, n_ext - 1u));
             uint64_t h[12];
 #pragma unroll
             for (int i = 0; i < 6; ++i) h[i] = q0[i], h[6 + i] = q1[i];
@@ -788,13 +797,14 @@ __global__ void __launch_bounds__(kFnvThreads) __attribute__((amdgpu_waves_per_e
                 }
                 if (!done) {
                     const uint64_t left = n_total - begin;
-                    from = gather_segment(a->map.ext, base, first, begin, left < kFnvLaneBytes ? left : kFnvLaneBytes);
+                    from = gather_segment(ext, base, first, begin, left < kFnvLaneBytes ? left : kFnvLaneBytes);
                 }
             }
             load_source(from, w);
         } else if (full) {
             load_segment(address_of(), w);
         }
+        if constexpr (kMapped) read_worth();
         // every load is issued before the first word is used: paired as they come, the first two loads' words had the others
         // wait for a memory round trip
         __builtin_amdgcn_sched_barrier(0);
