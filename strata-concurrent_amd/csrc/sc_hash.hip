@@ -107,7 +107,6 @@ __device__ __forceinline__ void renew_words(uint32_t (&w)[kFnvLaneBytes / 4]) {
 // ---- the sum on the matrix cores (what it computes and its weights: sc_hash_math.hpp) ----------------------------------
 __device__ const SumWeights g_sum_weights = sum_weights();
 constexpr int kWeightChunks = int(sizeof(SumWeights) / 16);
-static_assert(kWeightChunks % kFnvThreads == 0, "each lane stages whole chunks");
 __constant__ LanePow kLanePow = lane_pow();
 
 using i32x4 = __attribute__((ext_vector_type(4))) int32_t;
@@ -304,7 +303,8 @@ __global__ void __launch_bounds__(64) fnv_finish_kernel(const uint32_t* ctl, uin
 // live across the kernel would spill it and reload it from scratch, a memory round trip each time.
 __device__ __forceinline__ int lane_id() { return int(__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u))); }
 // Sleeps of 64 x 64 cycles before a look-back's first read of its window (the mapped kernel's last level writes its
-// gathered payload instead): 3.3 GB hashed in 1.36 ms with two, 1.38 with one or three
+// gathered payload instead): 3.3 GB hashed in 1.344 ms with two, 1.369 with one, and 0.48 GB in 249 us with two, 253 with
+// three (3.3 GB alike)
 constexpr int kFirstSleeps = 2, kFirstSleepsMapped = 0;
 constexpr uint32_t kSpinLimit = 1u << 16;   // reads of one window, about 0.2 s (sc_fnv1a64_set_spin_limit)
 // A bound the host sets only to test failure handling: every look-back of a workgroup after the first runs out at
@@ -365,17 +365,17 @@ __device__ __forceinline__ uint32_t start_byte() {
 
 // A workgroup's status word of one level: 0, kHasMap | map or kHasState | state.
 constexpr uint32_t kHasMap = 1u << 16, kHasState = 1u << 17;
-// The levels of a hash that looks back: two of four bits.  Each costs a wait of 6-7 us (see fnv_onepass_kernel), more than
-// the machines a third level saves (13.5 vector operations per two bytes with three levels of 3, 3 and 2 bits, 17 with two):
-// 3.3 GB in 1.36 against 1.41 ms, the 128K capture and hash in 1.76 against 1.89 ms.  A check given carries never waits
+// The levels of a hash that looks back: two of four bits.  Each costs 7-10 us from a workgroup's map to its start bits (see
+// fnv_onepass_kernel), more than the machines a third level saves (13.5 vector operations per two bytes with three levels of
+// 3, 3 and 2 bits, 17 with two): 3.3 GB in 1.36 against 1.41 ms, the 128K capture and hash in 1.76 against 1.89 ms.  A check given carries never waits
 // and takes the three levels: 0.87 against 1.02 ms.
 constexpr uint32_t kStatusWords = 2;
 
 // Workgroup g's start state at one level, run by one whole wave (the result is wave-uniform); the caller has published
 // g's map, and its end state is published after.  Lane l reads the status word of workgroup top - 64 + l; before workgroup
 // 0 stands the start state.  The maps after the nearest end state compose like those of a wave's lanes, so resolving a
-// window costs the same wherever that state lies.  Reading 128 or 256 words at once measured slower (1.66 and 1.87 ms for
-// 3.3 GB against 1.60: every read of a line that other XCDs write costs them all).
+// window costs the same wherever that state lies.  Reading 128 or 256 words at once measured slower (on a
+// form of the kernel that hashed 3.3 GB in 1.60 ms, 1.66 and 1.87: every read of a line that other XCDs write costs them all).
 template <int kLevel, int kJ, int kBits>
 __device__ __forceinline__ uint32_t look_back(uint32_t g, uint32_t map, int first_sleeps) {
     const int lane = lane_id();
@@ -651,11 +651,12 @@ __device__ __forceinline__ SegmentSource gather_segment(const HashExtent* ext, u
 
 // The wave's 16 KiB of gathered payload into the payload with coalesced stores: each lane holds 256 contiguous bytes,
 // so stores straight from the registers would put 64 lines under every store instruction (measured: the fused kernel
-// 3.3-3.7 ms with them against 2.3 ms without any store, and 8.2 ms with non-temporal ones).  Four passes of 4 KiB: a
-// quarter of the lanes write their segments into the wave's LDS rows (17 chunks apart, so the 16 writers of a
-// 16-byte column fall in different banks), then every lane reads back 16 bytes per 1 KiB and stores it, 1 KiB
-// contiguous per instruction, non-temporal.  Bytes at or past `limit` (the part hashed in the kernel) are not written
-// here.
+// 3.3-3.7 ms with them against 2.3 ms without any store, and 8.2 ms with non-temporal ones, in an earlier form).  Eight
+// passes of 2 KiB: an eighth of the lanes write their segments' step words into the wave's LDS rows (17 chunks apart), then
+// every lane reads back a chunk of step words and its partner, pairs them into a chunk of each half and stores the two: a
+// store instruction writes eight runs of 128 bytes, the first or the second halves of eight segments.  Non-temporal stores:
+// the 128K capture + hash 1.776 ms against 1.825 with regular ones, a paged 16381-token one 336 against 348 us.  Bytes at or
+// past `limit` (the part hashed in the kernel) are not written here.
 constexpr int kXposeRow = kFnvLaneBytes / 16 + 1;   // chunks per LDS row: a lane's 16 and one of padding
 __device__ __forceinline__ void store_wave(u32x4 (&lds)[8 * kXposeRow], const uint32_t (&w)[kFnvLaneBytes / 4],
                                            uint8_t* dst, uint64_t wave_begin, uint64_t limit, int lane) {
@@ -677,7 +678,6 @@ __device__ __forceinline__ void store_wave(u32x4 (&lds)[8 * kXposeRow], const ui
         const u32x4 b = {high_halves(lo.x, hi.x), high_halves(lo.y, hi.y), high_halves(lo.z, hi.z),
                          high_halves(lo.w, hi.w)};
         const uint64_t o = wave_begin + uint64_t(pass) * 2048u + uint64_t(seg) * kFnvLaneBytes + uint64_t(c) * 16u;
-        // non-temporal: the fused 128K capture 2.75 against 2.79-2.81 ms with regular stores
         if (o < limit) {   // whole segments: both chunks
             __builtin_nontemporal_store(a, (gu32x4*) (dst + o));
             __builtin_nontemporal_store(b, (gu32x4*) (dst + o + kPairBytes));
@@ -690,10 +690,11 @@ __device__ __forceinline__ void store_wave(u32x4 (&lds)[8 * kXposeRow], const ui
 
 // kMapped: the payload is gathered through `map` (stored, and hashed up to `n`, its whole lane segments) instead of read
 // from `data`.  Not kMapped, with `map.seg` set: the payload is read where its segments hold it (`data` unused).
-// What bounds it: the two look-backs of a workgroup's 35 us, 6-7 us each of waiting for the latest of the workgroups before
-// it (about 2 us), the word's way through memory and the read's (about 3.5 us), and, at 70% busy vector units, its 17
-// operations per two bytes.  3.3 GB in 1.36 ms (1.76 ms with three levels and the sums on the vector units), checked
-// with carries in 0.87 (1.29), the 128K slot gathered and hashed in 1.76 (2.03).
+// What bounds it: its 17 vector operations per two bytes, at 82% busy vector units, and the two look-backs, 9.9 and 7.5 us of
+// a workgroup's 33 from its map to its start bits (the maps' arithmetic, the wait for the latest of the workgroups before it
+// and the words' way through memory).  Given carries it neither waits nor takes tickets, and the vector units are 99% busy;
+// gathering, 62%, its reads and look-backs slowed by its own writes.  3.3 GB in 1.344 ms (1.76 ms with three levels and the
+// sums on the vector units), checked with carries in 0.87-0.88 (1.29), the 128K slot gathered and hashed in 1.776 (2.03).
 // Five waves per SIMD (96 VGPRs).  Taking several 64 KiB per workgroup, as the carried check does, measured slower here (3.3
 // GB in 1.60 ms): the workgroups' starts then spread over 3-5 us instead of 2, and every look-back waits for the latest.
 template <bool kMapped, bool kCarried>
@@ -915,7 +916,7 @@ FnvWorkspace fnv_workspace(uint64_t n) {
     return w;
 }
 
-// Clears a launch's words and enqueues the one-pass kernel over `a` (its ctl, status, groups, turns and spin limit set
+// Clears a launch's words and enqueues the one-pass kernel over `a` (its ctl, status, groups, pieces and spin limit set
 // here); returns ctl, or null for an empty input, which needs neither.
 template <bool kMapped>
 uint32_t* enqueue_onepass(OnepassArgs a, uint8_t* workspace, uint64_t bytes, hipStream_t stream) {
@@ -930,8 +931,10 @@ uint32_t* enqueue_onepass(OnepassArgs a, uint8_t* workspace, uint64_t bytes, hip
     hipLaunchKernelGGL(fnv_onepass_init_kernel, dim3(unsigned(init_blocks)), dim3(kThreads), 0, stream, a.status, words, a.ctl);
     if (!kMapped && a.carries.in) {
         // no workgroup waits for another: each takes up to four 64 KiB in turn, which spares it the start of a workgroup
-        // (3.3 GB checked in 0.88 ms against 1.35 ms with one each, and alike with eight) while others' kernels still get
-        // their turn on the CUs; fewer when that would leave some of the 1280 (five per CU) without work
+        // (3.3 GB checked in 0.884 ms against 0.907 with one each and 0.895 with eight) while others' kernels still get
+        // their turn on the CUs; fewer when that would leave some of the 1280 (five per CU) without work.  Between a few
+        // rounds of 1280 it costs the last round's idle CUs: 0.48 GB, 1838 workgroups of four, 155 us against 143 with one
+        // each
         const uint32_t turns = a.groups < 2 * 1280 ? 1 : a.groups < 4 * 1280 ? a.groups / 1280 : 4;
         hipLaunchKernelGGL((fnv_onepass_kernel<false, true>), dim3((a.groups + turns - 1) / turns), dim3(kFnvThreads), 0, stream, a);
     } else {

@@ -81,7 +81,7 @@ inline FastDiv make_fastdiv(uint32_t d) {
     return f;
 }
 
-// One row of the handoff table (device-resident, 72 bytes).
+// One row of the handoff table (device-resident, 80 bytes).
 struct MoveRow {
     int32_t kind;
     int32_t aux;            // kKv*: source tokens (rows past them are zero-filled); kConv: history rows
@@ -237,8 +237,9 @@ struct HashExtent {
     uint32_t page_chunks;    // pages: 16-byte chunks per page
 };
 static_assert(sizeof(HashExtent) == 48, "hash extents are 48 bytes");
-// Lanes of one hash workgroup: 256 (64 KiB) hashed 3.3 GB in 1.77 ms, against 4.84, 2.53 and 2.22 ms with 64, 128
-// and 512 (more workgroups mean more look-backs per byte, larger ones fewer resident workgroups per CU).
+// Lanes of one hash workgroup: 256 (64 KiB) hash 3.3 GB in 1.344 ms, against 2.55 and 1.52 ms with 128 and 512 (more
+// workgroups mean more look-backs per byte, larger ones fewer resident workgroups per CU); checked with carries 0.87 against
+// 0.90 and 0.97, gathered and hashed 1.78 against 2.88 and 1.88 (0.48 GB of pages: 0.338 against 0.466 and 0.326).
 constexpr int kFnvThreads = 256;
 constexpr int kFnvGroupBytes = kFnvThreads * kFnvLaneBytes;   // the payload bytes of one hash workgroup
 // The carries of a hashed input: the low byte of the running hash after each whole 64 KiB workgroup whose end lies
