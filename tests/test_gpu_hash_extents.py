@@ -1,6 +1,7 @@
 """The fused gather + hash over maps of many extents: each workgroup finds its first extent by sampling one end per share of
-the table and sampling again inside the share found.  Table sizes around one extent per share, one more sampling and two; extents of ragged lengths, some longer than a workgroup's 64 KiB, with gaps the map leaves as they are.
-Bytes and hash against numpy and the oracle's byte loop."""
+the table and sampling again inside the share found.  Table sizes around one extent per share, one more sampling and two;
+extents of ragged lengths, some longer than a workgroup's 64 KiB, with gaps the map leaves as they are.  Bytes and hash against
+numpy and the oracle's byte loop."""
 import numpy as np
 import pytest
 
